@@ -36,7 +36,8 @@ def hipcc():
 # one translation unit per medium's stage kernels plus the surrogate network's
 # kernels, compiled in parallel
 UNITS = ["cgfdh.hip", "stage_iso.hip", "stage_vti.hip", "stage_aniso.hip", "stage_visco.hip",
-         "surrogate.hip"]
+         "stage_tile_iso.hip", "stage_tile_vti.hip", "stage_tile_aniso.hip",
+         "stage_tile_visco.hip", "surrogate.hip"]
 
 
 def build_engine(verbose=False):

@@ -200,18 +200,23 @@ template <> struct Medium<MEDIUM_ANISO> {
                                         const float* Y, const float* Z) const
   {
 #pragma unroll
-    for (int t = 0; t < 6; t++) {
-      float acc = K(t, 0, m[0], m[1], m[2]) * X[0];
-      acc += K(t, 1, m[0], m[1], m[2]) * X[1];
-      acc += K(t, 2, m[0], m[1], m[2]) * X[2];
-      acc += K(t, 0, m[3], m[4], m[5]) * Y[0];
-      acc += K(t, 1, m[3], m[4], m[5]) * Y[1];
-      acc += K(t, 2, m[3], m[4], m[5]) * Y[2];
-      acc += K(t, 0, m[6], m[7], m[8]) * Z[0];
-      acc += K(t, 1, m[6], m[7], m[8]) * Z[1];
-      acc += K(t, 2, m[6], m[7], m[8]) * Z[2];
-      r[TXX + t] = acc;
-    }
+    for (int t = 0; t < 6; t++) hooke_row(t, r, m, X, Y, Z);
+  }
+
+  // row t of the stress rates
+  __device__ __forceinline__ void hooke_row(int t, float* r, const float* m, const float* X,
+                                            const float* Y, const float* Z) const
+  {
+    float acc = K(t, 0, m[0], m[1], m[2]) * X[0];
+    acc += K(t, 1, m[0], m[1], m[2]) * X[1];
+    acc += K(t, 2, m[0], m[1], m[2]) * X[2];
+    acc += K(t, 0, m[3], m[4], m[5]) * Y[0];
+    acc += K(t, 1, m[3], m[4], m[5]) * Y[1];
+    acc += K(t, 2, m[3], m[4], m[5]) * Y[2];
+    acc += K(t, 0, m[6], m[7], m[8]) * Z[0];
+    acc += K(t, 1, m[6], m[7], m[8]) * Z[1];
+    acc += K(t, 2, m[6], m[7], m[8]) * Z[2];
+    r[TXX + t] = acc;
   }
 
   // sv_curv_col_el_aniso.c:912-917

@@ -73,8 +73,9 @@ __global__ void metric_kernel(const float* __restrict__ xyz, float* __restrict__
 
 // ghost mirroring of the metric (gd_t.c:291-401): pass 0 mirrors x ghosts
 // for every (j,k), pass 1 y ghosts for every (i,k), pass 2 z ghosts for every
-// (i,j); run in that order as the reference does
-__global__ void metric_mirror_kernel(float* __restrict__ met, int pass, int nx, int ny, int nz,
+// (i,j); run in that order as the reference does.  nx: points of a row, px:
+// distance of two rows
+__global__ void metric_mirror_kernel(float* __restrict__ met, int pass, int nx, int px, int ny, int nz,
                                      int ni1, int ni2, int nj1, int nj2, int nk1, int nk2,
                                      long ss, long vol)
 {
@@ -86,20 +87,20 @@ __global__ void metric_mirror_kernel(float* __restrict__ met, int pass, int nx, 
     if (a >= ny) return;
     const int i = g < 3 ? g : ni2 + 1 + (g - 3);
     const int is = g < 3 ? 2 * ni1 - i - 1 : 2 * ni2 - i + 1;
-    dst = (long)i + (long)a * nx + (long)b * ss;
-    src = (long)is + (long)a * nx + (long)b * ss;
+    dst = (long)i + (long)a * px + (long)b * ss;
+    src = (long)is + (long)a * px + (long)b * ss;
   } else if (pass == 1) {
     if (a >= nx) return;
     const int j = g < 3 ? g : nj2 + 1 + (g - 3);
     const int js = g < 3 ? 2 * nj1 - j - 1 : 2 * nj2 - j + 1;
-    dst = (long)a + (long)j * nx + (long)b * ss;
-    src = (long)a + (long)js * nx + (long)b * ss;
+    dst = (long)a + (long)j * px + (long)b * ss;
+    src = (long)a + (long)js * px + (long)b * ss;
   } else {
     if (a >= nx) return;
     const int k = g < 3 ? g : nk2 + 1 + (g - 3);
     const int ks = g < 3 ? 2 * nk1 - k - 1 : 2 * nk2 - k + 1;
-    dst = (long)a + (long)b * nx + (long)k * ss;
-    src = (long)a + (long)b * nx + (long)ks * ss;
+    dst = (long)a + (long)b * px + (long)k * ss;
+    src = (long)a + (long)b * px + (long)ks * ss;
   }
   for (int m = 0; m < 10; m++) met[m * vol + dst] = met[m * vol + src];
 }

@@ -89,6 +89,9 @@ struct StageParams {
   const float* matVy;
   int npml;
   PmlDev pml[6];
+  int fslot[6];             // face -> index in pml, -1: no PML there
+  int fedge[6];             // last index from the low end / first to the high
+                            // end of each face's region along its normal
   float* aux_rhs_out[6];    // KIND_RHS only, per enabled face
   int nsrc;
   const SrcDev* src;
@@ -321,19 +324,18 @@ __device__ __forceinline__ void pml_aux_load(const PmlDev& F, long ia, float* a,
   }
 }
 
-// CFS-PML correction of one face (sv_curv_col_el_iso.c:645-1146) and the
-// RK combine of its auxiliary variables, from memory variables already
-// loaded; IDIM the face normal (0 x, 1 y, 2 z) as a template argument, so
-// that no register array is indexed by it
-template <int KIND, int MT, int IDIM>
-__device__ void pml_face_apply(const StageParams& P, const PmlDev& F, int fslot, int i, int j,
-                               int k, long ia, const float* Dd, const Medium<MT>& md, float slw,
-                               const float* m, float* r, const float* a, const float* apre,
-                               const float* aend)
+// CFS-PML correction of one face (sv_curv_col_el_iso.c:645-1146): the rates
+// r at a point corrected by the face's memory variables a, and their own
+// rates ah; cA, cB, cD the face's coefficients at the point; IDIM the face
+// normal (0 x, 1 y, 2 z) as a template argument, so that no register array
+// is indexed by it
+template <int MT, int IDIM>
+__device__ __forceinline__ void pml_face_rates(const StageParams& P, int i, int j, int k,
+                                               float cA, float cB, float cD, const float* Dd,
+                                               const Medium<MT>& md, float slw, const float* m,
+                                               float* r, const float* a, float* ah)
 {
   // m: the point's metric xi_x..zeta_z, already loaded by the caller
-  const int ic = IDIM == 0 ? i - F.i1 : (IDIM == 1 ? j - F.j1 : k - F.k1);
-  const float cD = F.D[ic], cA = F.A[ic], cB = F.B[ic];
   const float cBm1 = (float)((double)cB - 1.0);
   const float e1 = m[3 * IDIM], e2 = m[3 * IDIM + 1], e3 = m[3 * IDIM + 2];
   float rr[9];
@@ -341,7 +343,6 @@ __device__ void pml_face_apply(const StageParams& P, const PmlDev& F, int fslot,
   rr[VY] = slw * (e1 * Dd[TXY] + e2 * Dd[TYY] + e3 * Dd[TYZ]);
   rr[VZ] = slw * (e1 * Dd[TXZ] + e2 * Dd[TYZ] + e3 * Dd[TZZ]);
   md.one_dir(rr, e1, e2, e3, Dd);
-  float ah[9];
 #pragma unroll
   for (int c = 0; c < 9; c++) {
     r[c] += cBm1 * rr[c] - cB * a[c];
@@ -364,6 +365,19 @@ __device__ void pml_face_apply(const StageParams& P, const PmlDev& F, int fslot,
       ah[c] += cD * s[c];
     }
   }
+}
+
+// the correction and the RK combine of the face's memory variables, from
+// memory variables already loaded
+template <int KIND, int MT, int IDIM>
+__device__ void pml_face_apply(const StageParams& P, const PmlDev& F, int fslot, int i, int j,
+                               int k, long ia, const float* Dd, const Medium<MT>& md, float slw,
+                               const float* m, float* r, const float* a, const float* apre,
+                               const float* aend)
+{
+  const int ic = IDIM == 0 ? i - F.i1 : (IDIM == 1 ? j - F.j1 : k - F.k1);
+  float ah[9];
+  pml_face_rates<MT, IDIM>(P, i, j, k, F.A[ic], F.B[ic], F.D[ic], Dd, md, slw, m, r, a, ah);
   if (KIND == KIND_RHS) {
 #pragma unroll
     for (int c = 0; c < 9; c++) P.aux_rhs_out[fslot][c * F.fn + ia] = ah[c];
@@ -570,9 +584,12 @@ __device__ __forceinline__ void combine_store(const StageParams& P, long p, cons
 // memory-variable rates into r[9 + 6n + {xx,yy,zz,yz,xz,xy}] and the memory
 // terms subtracted from the stress rates, with the reference's double
 // intermediates
-__device__ __forceinline__ void atten(const StageParams& P, long p, float lam, float mu, float* r)
+// w(c): component c of the level at the point, y: Ylam_n, Ymu_n there; NB:
+// bodies r and y have room for
+template <int NB, class W>
+__device__ __forceinline__ void atten(const StageParams& P, const W& w, const float* y, float lam,
+                                      float mu, float* r)
 {
-  const long V = P.vol;
   const float hTxx = r[TXX], hTyy = r[TYY], hTzz = r[TZZ];
   const float hTxy = r[TXY], hTxz = r[TXZ], hTyz = r[TYZ];
   const float sum_hxyz = (hTxx + hTyy + hTzz) / (3 * lam + 2 * mu);
@@ -586,11 +603,11 @@ __device__ __forceinline__ void atten(const StageParams& P, long p, float lam, f
   float sJxyz = 0.0f, sJxx = 0.0f, sJyy = 0.0f, sJzz = 0.0f, sJxy = 0.0f, sJxz = 0.0f,
         sJyz = 0.0f;
 #pragma unroll
-  for (int n = 0; n < MAXWELL_MAX; n++) {
+  for (int n = 0; n < NB; n++) {
     if (n >= P.nmax) break;
-    const float* J = P.wcur + (9 + 6 * n) * V + p;
-    const float Jxx = J[0], Jyy = J[V], Jzz = J[2 * V], Jyz = J[3 * V], Jxz = J[4 * V],
-                Jxy = J[5 * V];
+    const int c = 9 + 6 * n;
+    const float Jxx = w(c), Jyy = w(c + 1), Jzz = w(c + 2), Jyz = w(c + 3), Jxz = w(c + 4),
+                Jxy = w(c + 5);
     const float wl = P.wl[n];
     float* h = r + 9 + 6 * n;
     h[0] = wl * (EVxx - Jxx);
@@ -599,8 +616,7 @@ __device__ __forceinline__ void atten(const StageParams& P, long p, float lam, f
     h[3] = wl * (EVyz - Jyz);
     h[4] = wl * (EVxz - Jxz);
     h[5] = wl * (EVxy - Jxy);
-    const float Yl = ld_stream(P.ylam + (2 * n) * V + p);
-    const float Ym = ld_stream(P.ylam + (2 * n + 1) * V + p);
+    const float Yl = y[2 * n], Ym = y[2 * n + 1];
     sJxyz += Yl * (Jxx + Jyy + Jzz);
     sJxx += Ym * Jxx;
     sJyy += Ym * Jyy;
@@ -615,6 +631,17 @@ __device__ __forceinline__ void atten(const StageParams& P, long p, float lam, f
   r[TXY] = hTxy - (float)(2.0 * mu * sJxy);
   r[TXZ] = hTxz - (float)(2.0 * mu * sJxz);
   r[TYZ] = hTyz - (float)(2.0 * mu * sJyz);
+}
+
+__device__ __forceinline__ void atten(const StageParams& P, long p, float lam, float mu, float* r)
+{
+  float y[2 * MAXWELL_MAX];
+#pragma unroll
+  for (int n = 0; n < 2 * MAXWELL_MAX; n++) {
+    if (n >= 2 * P.nmax) break;
+    y[n] = ld_stream(P.ylam + n * P.vol + p);
+  }
+  atten<MAXWELL_MAX>(P, [&](int c) { return P.wcur[c * P.vol + p]; }, y, lam, mu, r);
 }
 
 // the interior form of everything after the derivatives: momentum, Hooke's

@@ -18,8 +18,9 @@
 // combine inputs after the arithmetic) plus the shell; 14 the LDS-tiled
 // plane kernel (64x8) with the same phased loads plus the shell; 15 variant
 // 12 compiled for 3 waves per SIMD (a few registers spill) plus the shell;
-// 16 the two-phase kernel over whole rows with the PML faces folded in, the
-// free-surface rows on the general kernel; 17 the two-phase interior kernel
+// 16 whole rows with the PML faces folded in, the free-surface rows on the
+// general kernel: the tile kernel (stage_tile.h) steps, the two-phase kernel
+// evaluates a single right-hand side and serves volumes past 32-bit offsets; 17 the two-phase interior kernel
 // on the tiles clear of every PML face and the phased shell kernel on the
 // PML slabs (x edges in whole 64-point tiles, y and z slabs in whole rows),
 // free-surface rows on the general kernel.
@@ -48,8 +49,9 @@ struct LaunchCtx {
   int tgx, tgy;            // tile group of the grouped block order (0: default)
   int merge_shell;         // 1: the five PML slabs of the shell in one launch
   hipStream_t shell_stream;  // stream of the shell boxes (= stream, or one beside it)
-  int slab_only;           // variant 16: launch only the free-surface rows (the batch's
-                           // fused launch runs the whole rows of every grid)
+  int slab_only;           // variant 16: launch only the free-surface rows (the tile
+                           // kernel, or the batch's fused launch, runs the others)
+  long bytes;              // of the solver's volumes
 };
 
 // the whole-row box of variant 16 with its block grouping resolved; returns
@@ -282,6 +284,12 @@ void launch_rows_multi_mt(hipStream_t st, const RowsMulti& R, int nblocks, int k
     default: launch_rows_multi<KIND_LAST, MT, 4>(st, R, nblocks, code); break;
   }
 }
+
+// the whole rows of variant 16, defined in stage_tile_<medium>.hip
+void launch_tile_iso(const LaunchCtx& L, const StageParams& P, int kind, int dx, int dy, int dz);
+void launch_tile_vti(const LaunchCtx& L, const StageParams& P, int kind, int dx, int dy, int dz);
+void launch_tile_aniso(const LaunchCtx& L, const StageParams& P, int kind, int dx, int dy, int dz);
+void launch_tile_visco(const LaunchCtx& L, const StageParams& P, int kind, int dx, int dy, int dz);
 
 // defined in stage_iso.hip, stage_vti.hip and stage_aniso.hip
 void launch_stage_iso(const LaunchCtx& L, const StageParams& P, int kind, int dx, int dy, int dz);
