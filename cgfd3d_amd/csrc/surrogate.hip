@@ -11,6 +11,7 @@
 
 #include <cstdint>
 #include <cstdio>
+#include <type_traits>
 
 #include "cgfdh.h"
 #include "cgfds.h"
@@ -56,121 +57,188 @@ struct GemmArgs {
   long ldc16;
   int kchunk;             // K range per blockIdx.z, multiple of 32
   float* work;            // split-K partials [gridDim.z][M][N] (then no epilogue)
+  int vec16;              // mask and C16 rows allow 8-byte accesses
 };
 
 enum { EPI_NONE = 0, EPI_RELU = 1, EPI_MASK = 2 };
 
-constexpr int BM = 64, BN = 64, BK = 32, LDK = BK + 8;   // LDS rows padded by 16 B
+// ---------------------------------------------------------------------------
+// GEMM
+// ---------------------------------------------------------------------------
+
+typedef short s16x4 __attribute__((ext_vector_type(4)));
+typedef float f32x4u __attribute__((ext_vector_type(4), aligned(4)));
+typedef uint16_t u16x4 __attribute__((ext_vector_type(4)));
+
+constexpr unsigned OUT = ~15u;   // an offset past every operand: loads zeros
+
+// One operand's tile, loaded straight to LDS 16 bytes a lane.  KC: the
+// contraction index is the contiguous one, R rows of BK; otherwise BK rows of R.
+// Inside a row the 16-byte chunks are exchanged by an exclusive or with bits of
+// the row, so that the 16 rows (KC) or the 4 x 2 rows (not KC) a fragment reads
+// at one chunk lie in different banks.
+template <bool KC, int R, int BK, int NT> struct Operand {
+  static constexpr int ROWS = KC ? R : BK, COLS = KC ? BK : R;
+  static constexpr int CH = COLS / 8;             // chunks of a row
+  static constexpr int N = ROWS * CH / NT;        // loads of a thread
+  static_assert(ROWS * CH % NT == 0 && (CH & (CH - 1)) == 0, "");
+  static __device__ __forceinline__ int swz(int r)
+  {
+    if (KC) return r & (CH < 8 ? CH - 1 : 7);
+    return ((r & 3) << 1 & (CH - 1)) ^ (CH >= 16 ? (r >> 3 & 1) << 3 : 0);
+  }
+
+  // the tile at contraction index k of the operand whose first row (KC) or
+  // column is r0 of nr
+  static __device__ __forceinline__ void load(const uint16_t* base, long ld, int r0, int nr, int k,
+                                              int ke, uint16_t* lds)
+  {
+    const uint16_t* p = base + (KC ? (long)r0 * ld + k : (long)k * ld + r0);
+    const int t = threadIdx.x, w = __builtin_amdgcn_readfirstlane(t >> 6);
+#pragma unroll
+    for (int i = 0; i < N; ++i) {
+      // the wave's first row by scalar arithmetic, the lanes' distance to it (at
+      // most 16 rows) in the 32-bit offset
+      const int rw = (i * NT + w * 64) / CH;
+      const int id = i * NT + t, r = id / CH, c = (id % CH) ^ swz(r);
+      const __amdgpu_buffer_rsrc_t q = __builtin_amdgcn_make_buffer_rsrc(
+          (void*)(p + rw * ld), 0, (int)0xfffffff0, 0x00020000);
+      const bool ok = KC ? (r0 + r < nr && k + 8 * c < ke) : (k + r < ke && r0 + 8 * c < nr);
+      const unsigned off = ok ? (unsigned)((r - rw) * (unsigned)ld + 8 * c) * 2u : OUT;
+      __builtin_amdgcn_raw_ptr_buffer_load_lds(
+          q, (__attribute__((address_space(3))) void*)(lds + (long)(i * NT + w * 64) * 8), 16,
+          (int)off, 0, 0, 0);
+    }
+  }
+
+  // the MFMA fragment of rows r .. r+15 at contraction indices kk .. kk+31:
+  // lane l holds row l%16, k = 8*(l/16) .. +7
+  static __device__ __forceinline__ bf16x8 frag(const uint16_t* lds, int r, int kk)
+  {
+    const int l = threadIdx.x & 63, l16 = l & 15, g = l >> 4;
+    if (KC) {
+      const int row = r + l16;
+      return *(const bf16x8*)(lds + (row * CH + (((kk >> 3) + g) ^ swz(row))) * 8);
+    }
+    // the transposing read gives each lane of 16 one column of the 4 rows of
+    // 16 that they address together
+    const int k = kk + 8 * g + (l16 >> 2), col = r + 4 * (l16 & 3);
+    const uint16_t* a = lds + (k * CH + ((col >> 3) ^ swz(k))) * 8 + (col & 7);
+    union {
+      s16x4 h[2];
+      bf16x8 v;
+    } u;
+    typedef __attribute__((address_space(3))) s16x4* lp;
+    u.h[0] = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lp)a);
+    u.h[1] = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lp)(a + 4 * CH * 8));
+    return u.v;
+  }
+};
 
 // C[M][N] = sum_k opA[m][k] * opB[k][n].  opA = A ([M][K]) or, TA, A^T with A
 // stored [K][M]; opB = B ([K][N]) or, TB, B^T with B stored [N][K].
-// 256 threads = 4 waves in a 2x2 arrangement, each wave a 32x32 sub-tile of
-// 2x2 MFMA 16x16x32 tiles.  Tiles go through LDS as [row][k] with k
-// contiguous, double buffered with one barrier per K step.
-template <int TA, int TB>
-__global__ __launch_bounds__(256) void gemm_bf16_kernel(GemmArgs g)
+// WM x WN waves over a BM x BN tile, each BM/WM x BN/WN in MFMA 16x16x32 tiles;
+// NS stages of BK in a ring, NS - 1 of them in flight.  The products are formed
+// as (B^T A^T): a lane then holds 4 neighbouring columns of one row of C, which
+// leave in one 16- or 8-byte store.
+template <int TA, int TB, int BM, int BN, int BK, int NS, int WM, int WN>
+__global__ __launch_bounds__(64 * WM * WN) void gemm_bf16_kernel(GemmArgs g)
 {
-  __shared__ __attribute__((aligned(16))) uint16_t As[2][BM][LDK];
-  __shared__ __attribute__((aligned(16))) uint16_t Bs[2][BN][LDK];
-  const int t = threadIdx.x, lane = t & 63, w = t >> 6;
+  constexpr int NT = 64 * WM * WN;
+  using OA = Operand<!TA, BM, BK, NT>;
+  using OB = Operand<TB, BN, BK, NT>;
+  constexpr int FM = BM / WM / 16, FN = BN / WN / 16;
+  __shared__ __attribute__((aligned(16))) uint16_t As[NS][BM * BK];
+  __shared__ __attribute__((aligned(16))) uint16_t Bs[NS][BN * BK];
+  const int lane = threadIdx.x & 63, w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int m0 = blockIdx.x * BM, n0 = blockIdx.y * BN;
   const int kb = blockIdx.z * g.kchunk;
   const int ke = min(g.K, kb + g.kchunk);
-  const int wm = (w >> 1) * 32, wn = (w & 1) * 32;
+  const int wm = w / WN * (BM / WM), wn = w % WN * (BN / WN);
+  // columns of 16 this wave has to form
+  const int nj = min(FN, (g.N - n0 - wn + 15) / 16);
 
-  // global -> register staging: each thread moves 8 bf16 (16 B) of A and of B
-  const int a_r = TA ? (t >> 3) : (t >> 2);          // k row (TA) or m row
-  const int a_c = TA ? (t & 7) * 8 : (t & 3) * 8;    // m col (TA) or k col
-  const int b_r = TB ? (t >> 2) : (t >> 3);          // n row (TB) or k row
-  const int b_c = TB ? (t & 3) * 8 : (t & 7) * 8;    // k col (TB) or n col
-  uint4 ra, rb;
-  auto gload = [&](int k0) {
-    const uint4 z = {0u, 0u, 0u, 0u};
-    if (TA) {
-      const int k = k0 + a_r, m = m0 + a_c;
-      ra = (k < ke && m < g.M) ? *(const uint4*)(g.A + (long)k * g.lda + m) : z;
-    } else {
-      const int m = m0 + a_r, k = k0 + a_c;
-      ra = (k < ke && m < g.M) ? *(const uint4*)(g.A + (long)m * g.lda + k) : z;
-    }
-    if (TB) {
-      const int n = n0 + b_r, k = k0 + b_c;
-      rb = (k < ke && n < g.N) ? *(const uint4*)(g.B + (long)n * g.ldb + k) : z;
-    } else {
-      const int k = k0 + b_r, n = n0 + b_c;
-      rb = (k < ke && n < g.N) ? *(const uint4*)(g.B + (long)k * g.ldb + n) : z;
-    }
+  f32x4 acc[FM][FN];
+#pragma unroll
+  for (int i = 0; i < FM; ++i)
+#pragma unroll
+    for (int j = 0; j < FN; ++j) acc[i][j] = (f32x4){0.f, 0.f, 0.f, 0.f};
+
+  const int nk = (ke - kb + BK - 1) / BK;
+  auto load = [&](int s) {
+    // past the end the loads bring zeros, so that every turn waits for as many
+    OA::load(g.A, g.lda, m0, g.M, kb + s * BK, s < nk ? ke : 0, As[s % NS]);
+    OB::load(g.B, g.ldb, n0, g.N, kb + s * BK, s < nk ? ke : 0, Bs[s % NS]);
   };
-  auto lstore = [&](int buf) {
-    if (TA) {
-      const uint16_t* e = (const uint16_t*)&ra;
 #pragma unroll
-      for (int q = 0; q < 8; ++q) As[buf][a_c + q][a_r] = e[q];
-    } else {
-      *(uint4*)&As[buf][a_r][a_c] = ra;
-    }
-    if (TB) {
-      *(uint4*)&Bs[buf][b_r][b_c] = rb;
-    } else {
-      const uint16_t* e = (const uint16_t*)&rb;
+  for (int s = 0; s < NS - 1; ++s) load(s);
+  for (int s = 0; s < nk; ++s) {
+    load(s + NS - 1);
+    asm volatile("s_waitcnt vmcnt(%0)\n\ts_barrier" ::"n"((NS - 1) * (OA::N + OB::N)) : "memory");
+    const uint16_t *pa = As[s % NS], *pb = Bs[s % NS];
 #pragma unroll
-      for (int q = 0; q < 8; ++q) Bs[buf][b_c + q][b_r] = e[q];
-    }
-  };
-
-  f32x4 acc[2][2];
+    for (int kk = 0; kk < BK; kk += 32) {
+      bf16x8 a[FM], b[FN];
 #pragma unroll
-  for (int i = 0; i < 2; ++i)
+      for (int i = 0; i < FM; ++i) a[i] = OA::frag(pa, wm + 16 * i, kk);
 #pragma unroll
-    for (int j = 0; j < 2; ++j) acc[i][j] = (f32x4){0.f, 0.f, 0.f, 0.f};
-
-  // lane l feeds row/col l%16 of its 16x16 tile with k = 8*(l/16) .. +7
-  const int lr = lane & 15, lk = (lane >> 4) * 8;
-  int buf = 0;
-  if (kb < ke) {
-    gload(kb);
-    lstore(0);
-  }
-  __syncthreads();
-  for (int k0 = kb; k0 < ke; k0 += BK) {
-    const bool more = k0 + BK < ke;
-    if (more) gload(k0 + BK);
-    bf16x8 a[2], b[2];
+      for (int j = 0; j < FN; ++j)
+        if (j < nj) b[j] = OB::frag(pb, wn + 16 * j, kk);
 #pragma unroll
-    for (int i = 0; i < 2; ++i) a[i] = *(const bf16x8*)&As[buf][wm + 16 * i + lr][lk];
+      for (int j = 0; j < FN; ++j)
+        if (j < nj) {
 #pragma unroll
-    for (int j = 0; j < 2; ++j) b[j] = *(const bf16x8*)&Bs[buf][wn + 16 * j + lr][lk];
-#pragma unroll
-    for (int i = 0; i < 2; ++i)
-#pragma unroll
-      for (int j = 0; j < 2; ++j)
-        acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[i], b[j], acc[i][j], 0, 0, 0);
-    if (more) lstore(buf ^ 1);
-    __syncthreads();
-    buf ^= 1;
-  }
-
-  // D layout of a 16x16 MFMA tile: lane l holds rows 4*(l/16)+e, column l%16
-#pragma unroll
-  for (int i = 0; i < 2; ++i)
-#pragma unroll
-    for (int j = 0; j < 2; ++j)
-#pragma unroll
-      for (int e = 0; e < 4; ++e) {
-        const int r = m0 + wm + 16 * i + 4 * (lane >> 4) + e;
-        const int c = n0 + wn + 16 * j + lr;
-        if (r >= g.M || c >= g.N) continue;
-        float v = acc[i][j][e];
-        if (g.work) {
-          g.work[((long)blockIdx.z * g.M + r) * g.N + c] = v;
-          continue;
+          for (int i = 0; i < FM; ++i)
+            acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(b[j], a[i], acc[i][j], 0, 0, 0);
         }
-        if (g.bias) v = v + g.bias[c];
-        if (g.epi == EPI_RELU) v = v > 0.f ? v : 0.f;
-        if (g.epi == EPI_MASK) v = bf_pos(g.mask[(long)r * g.ldm + c]) ? v : 0.f;
-        if (g.C32) g.C32[(long)r * g.ldc32 + c] = v;
-        if (g.C16) g.C16[(long)r * g.ldc16 + c] = f2bf(v);
+    }
+    // the stage is read before it is loaded again
+    asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
+  }
+
+  // D layout of a 16x16 MFMA tile: lane l holds rows (here columns of C)
+  // 4*(l/16)+e, column (row of C) l%16
+#pragma unroll
+  for (int j = 0; j < FN; ++j) {
+    const int c = n0 + wn + 16 * j + 4 * (lane >> 4);
+    if (c >= g.N) continue;          // N is a multiple of 8: all four or none
+    f32x4 bias = {0.f, 0.f, 0.f, 0.f};
+    if (g.bias && !g.work) bias = *(const f32x4u*)(g.bias + c);
+#pragma unroll
+    for (int i = 0; i < FM; ++i) {
+      const int r = m0 + wm + 16 * i + (lane & 15);
+      if (r >= g.M) continue;
+      f32x4 v = acc[i][j];
+      if (g.work) {
+        *(f32x4u*)(g.work + ((long)blockIdx.z * g.M + r) * g.N + c) = v;
+        continue;
       }
+      if (g.bias) v = v + bias;
+      if (g.epi == EPI_RELU) {
+#pragma unroll
+        for (int e = 0; e < 4; ++e) v[e] = v[e] > 0.f ? v[e] : 0.f;
+      }
+      if (g.epi == EPI_MASK) {
+        u16x4 h;
+        const uint16_t* q = g.mask + (long)r * g.ldm + c;
+        if (g.vec16) h = *(const u16x4*)q;
+        else
+          for (int e = 0; e < 4; ++e) h[e] = q[e];
+#pragma unroll
+        for (int e = 0; e < 4; ++e) v[e] = bf_pos(h[e]) ? v[e] : 0.f;
+      }
+      if (g.C32) *(f32x4u*)(g.C32 + (long)r * g.ldc32 + c) = v;
+      if (g.C16) {
+        u16x4 h;
+#pragma unroll
+        for (int e = 0; e < 4; ++e) h[e] = f2bf(v[e]);
+        uint16_t* q = g.C16 + (long)r * g.ldc16 + c;
+        if (g.vec16) *(u16x4*)q = h;
+        else
+          for (int e = 0; e < 4; ++e) q[e] = h[e];
+      }
+    }
+  }
 }
 
 // out[r][c] = sum over s of work[s][r][c], s in increasing order (deterministic)
@@ -345,23 +413,47 @@ extern "C" int cgfds_gemm_bf16(int M, int N, int K, const void* A, long lda, int
     return sfail(CGFDH_EINVAL, "cgfds_gemm_bf16: bad epilogue or missing mask");
   if (splitk < 1 || splitk > 1024)
     return sfail(CGFDH_EINVAL, "cgfds_gemm_bf16: splitk outside 1..1024");
-  int kchunk = ((K + splitk - 1) / splitk + BK - 1) / BK * BK;
+  int kchunk = ((K + splitk - 1) / splitk + 31) / 32 * 32;
   int S = (K + kchunk - 1) / kchunk;
   if (S > 1 && (!work || !C32 || C16 || bias || epilogue != EPI_NONE))
     return sfail(CGFDH_EINVAL,
                  "cgfds_gemm_bf16: split-K needs a work buffer, FP32 output and no epilogue");
+  auto al8 = [](const void* p, long ld) { return !p || (((uintptr_t)p & 7u) == 0 && ld % 4 == 0); };
   GemmArgs g{M, N, K, (const uint16_t*)A, lda, (const uint16_t*)B, ldb, bias, epilogue,
              (const uint16_t*)mask, ldm, C32, ldc32, (uint16_t*)C16, ldc16, kchunk,
-             S > 1 ? work : nullptr};
+             S > 1 ? work : nullptr, al8(mask, ldm) && al8(C16, ldc16)};
   hipStream_t st = (hipStream_t)stream;
-  // row tiles on x (up to 2^31 - 1 blocks), column tiles on y
-  dim3 grid((M + BM - 1) / BM, (N + BN - 1) / BN, S);
-  if (grid.y > 65535)
+  if ((N + 63) / 64 > 65535)
     return sfail(CGFDH_EINVAL, "cgfds_gemm_bf16: N above 65535*64 columns");
-  if (!transA && !transB) hipLaunchKernelGGL((gemm_bf16_kernel<0, 0>), grid, dim3(256), 0, st, g);
-  if (!transA && transB) hipLaunchKernelGGL((gemm_bf16_kernel<0, 1>), grid, dim3(256), 0, st, g);
-  if (transA && !transB) hipLaunchKernelGGL((gemm_bf16_kernel<1, 0>), grid, dim3(256), 0, st, g);
-  if (transA && transB) hipLaunchKernelGGL((gemm_bf16_kernel<1, 1>), grid, dim3(256), 0, st, g);
+  const int form = (transA ? 2 : 0) + (transB ? 1 : 0);
+  // row tiles on x (up to 2^31 - 1 blocks), column tiles on y
+  auto launch = [&](auto bm, auto bn, auto bk, auto ns, auto wm, auto wn) {
+    constexpr int BM = decltype(bm)::value, BN = decltype(bn)::value, BK = decltype(bk)::value,
+                  NS = decltype(ns)::value, WM = decltype(wm)::value, WN = decltype(wn)::value;
+    const dim3 grid((M + BM - 1) / BM, (N + BN - 1) / BN, S), blk(64 * WM * WN);
+    switch (form) {
+    case 0: hipLaunchKernelGGL((gemm_bf16_kernel<0, 0, BM, BN, BK, NS, WM, WN>), grid, blk, 0, st, g); break;
+    case 1: hipLaunchKernelGGL((gemm_bf16_kernel<0, 1, BM, BN, BK, NS, WM, WN>), grid, blk, 0, st, g); break;
+    case 2: hipLaunchKernelGGL((gemm_bf16_kernel<1, 0, BM, BN, BK, NS, WM, WN>), grid, blk, 0, st, g); break;
+    default: hipLaunchKernelGGL((gemm_bf16_kernel<1, 1, BM, BN, BK, NS, WM, WN>), grid, blk, 0, st, g); break;
+    }
+  };
+#define CGFDS_I(n) std::integral_constant<int, n>{}
+  // The largest tile that still leaves a block for each of the 256 compute
+  // units: fewer bytes through LDS a product.  us, 128 x 128 and 64 x 64:
+  // 2048 x 4096 x 512 (512 large tiles) 23, 31; 2048 x 512 x 512 (64) 16, 9.
+  // Where even 64 x 64 leaves units idle the contraction is a serial chain, so
+  // fewer, deeper stages and twice the tiles: 64 x 512 x 4096 28, 37; 512 x 512
+  // x 4096 34, 51; level with 64 x 64 at K = 512 and below.
+  const long big = (long)((M + 127) / 128) * ((N + 127) / 128) * S;
+  const long mid = (long)((M + 63) / 64) * ((N + 63) / 64) * S;
+  if (big >= 256)
+    launch(CGFDS_I(128), CGFDS_I(128), CGFDS_I(64), CGFDS_I(2), CGFDS_I(2), CGFDS_I(2));
+  else if (mid >= 256)
+    launch(CGFDS_I(64), CGFDS_I(64), CGFDS_I(64), CGFDS_I(3), CGFDS_I(2), CGFDS_I(2));
+  else
+    launch(CGFDS_I(64), CGFDS_I(32), CGFDS_I(128), CGFDS_I(4), CGFDS_I(2), CGFDS_I(2));
+#undef CGFDS_I
   if (int rc = launch_check("cgfds_gemm_bf16")) return rc;
   if (S > 1) {
     long n = (long)M * N;
