@@ -7,6 +7,7 @@
 // Storage: bf16 values are raw 16-bit words (upper half of an IEEE binary32,
 // round-to-nearest-even on conversion); matrices are row-major with explicit
 // leading dimensions in elements.
+#include <algorithm>
 #include <hip/hip_runtime.h>
 
 #include <cstdint>
@@ -57,8 +58,42 @@ struct GemmArgs {
   long ldc16;
   int kchunk;             // K range per blockIdx.z, multiple of 32
   float* work;            // split-K partials [gridDim.z][M][N] (then no epilogue)
-  int vec16;              // mask and C16 rows allow 8-byte accesses
+  int vec16;              // mask and C16 rows allow 16-byte accesses
+  int order, mt, nt, S;   // block order (below), row and column tiles, K splits
+  // column sums of B (opA transposed, B not: the bias gradient beside the
+  // weight gradient): [N], or with work its partials behind the products'
+  float* csum;
+  // moment-tensor contraction of the rows (N <= BN): y[r][t][c] = sum over k of
+  // mten[r / rps][k] * C[r][t][k][c], k below nk, c below nc
+  const float* mten;
+  float* y;
+  int nk, nc, rps;
 };
+
+// The order of the blocks.  Blocks go to the 8 XCDs in turn, each with its own
+// L2, and those that read the same rows belong on one of them, close together:
+// ORD_ROWS the column tiles of a row tile, ORD_SPLIT all tiles of one range of
+// the contraction.
+enum { ORD_PLAIN = 0, ORD_ROWS = 1, ORD_SPLIT = 2 };
+
+__device__ __forceinline__ bool gemm_tile(const GemmArgs& g, int& x, int& y, int& z)
+{
+  const unsigned f = blockIdx.x, q = f / 8, xcd = f % 8;
+  if (g.order == ORD_ROWS) {
+    x = q / g.nt * 8 + xcd;
+    y = q % g.nt;
+    z = 0;
+    return x < g.mt;
+  }
+  const unsigned tiles = (unsigned)g.mt * g.nt;
+  const unsigned t = g.order == ORD_SPLIT ? q % tiles : f % tiles;
+  z = g.order == ORD_SPLIT ? q / tiles * 8 + xcd : f / tiles;
+  x = t % g.mt;
+  y = t / g.mt;
+  return z < g.S;
+}
+
+constexpr int MT_MAX = 8;   // basis terms of a moment-tensor output
 
 enum { EPI_NONE = 0, EPI_RELU = 1, EPI_MASK = 2 };
 
@@ -69,6 +104,7 @@ enum { EPI_NONE = 0, EPI_RELU = 1, EPI_MASK = 2 };
 typedef short s16x4 __attribute__((ext_vector_type(4)));
 typedef float f32x4u __attribute__((ext_vector_type(4), aligned(4)));
 typedef uint16_t u16x4 __attribute__((ext_vector_type(4)));
+typedef uint16_t u16x8 __attribute__((ext_vector_type(8)));
 
 constexpr unsigned OUT = ~15u;   // an offset past every operand: loads zeros
 
@@ -148,15 +184,26 @@ __global__ __launch_bounds__(64 * WM * WN) void gemm_bf16_kernel(GemmArgs g)
   using OA = Operand<!TA, BM, BK, NT>;
   using OB = Operand<TB, BN, BK, NT>;
   constexpr int FM = BM / WM / 16, FN = BN / WN / 16;
-  __shared__ __attribute__((aligned(16))) uint16_t As[NS][BM * BK];
-  __shared__ __attribute__((aligned(16))) uint16_t Bs[NS][BN * BK];
+  // the ring; behind the products the waves' output rows
+  constexpr int RING = NS * (BM + BN) * BK, ROWS = BM * BN + 8 * BM * WN;
+  __shared__ __attribute__((aligned(16))) uint16_t sm[RING > ROWS ? RING : ROWS];
+  uint16_t *const As = sm, *const Bs = sm + NS * BM * BK;
   const int lane = threadIdx.x & 63, w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-  const int m0 = blockIdx.x * BM, n0 = blockIdx.y * BN;
-  const int kb = blockIdx.z * g.kchunk;
+  int tx, ty, tz;
+  if (!gemm_tile(g, tx, ty, tz)) return;
+  const int m0 = tx * BM, n0 = ty * BN;
+  const int kb = tz * g.kchunk;
   const int ke = min(g.K, kb + g.kchunk);
   const int wm = w / WN * (BM / WM), wn = w % WN * (BN / WN);
   // columns of 16 this wave has to form
   const int nj = min(FN, (g.N - n0 - wn + 15) / 16);
+  // the waves of the first row tile that form the column sums of B
+  const bool cs = TA && !TB && g.csum && m0 == 0 && wm == 0;
+  f32x4 sums[FN];
+  const bf16x8 ones = {(__bf16)1.f, (__bf16)1.f, (__bf16)1.f, (__bf16)1.f,
+                       (__bf16)1.f, (__bf16)1.f, (__bf16)1.f, (__bf16)1.f};
+#pragma unroll
+  for (int j = 0; j < FN; ++j) sums[j] = (f32x4){0.f, 0.f, 0.f, 0.f};
 
   f32x4 acc[FM][FN];
 #pragma unroll
@@ -166,16 +213,35 @@ __global__ __launch_bounds__(64 * WM * WN) void gemm_bf16_kernel(GemmArgs g)
 
   const int nk = (ke - kb + BK - 1) / BK;
   auto load = [&](int s) {
-    // past the end the loads bring zeros, so that every turn waits for as many
-    OA::load(g.A, g.lda, m0, g.M, kb + s * BK, s < nk ? ke : 0, As[s % NS]);
-    OB::load(g.B, g.ldb, n0, g.N, kb + s * BK, s < nk ? ke : 0, Bs[s % NS]);
+    OA::load(g.A, g.lda, m0, g.M, kb + s * BK, ke, As + s % NS * (BM * BK));
+    OB::load(g.B, g.ldb, n0, g.N, kb + s * BK, ke, Bs + s % NS * (BN * BK));
   };
+  // what the epilogue adds is requested before the products: asked for behind
+  // them it is a chain of latencies, longer than a short contraction itself
+  f32x4 bias[FN];
 #pragma unroll
-  for (int s = 0; s < NS - 1; ++s) load(s);
+  for (int j = 0; j < FN; ++j) {
+    const int c = n0 + wn + 16 * j + 4 * (lane >> 4);
+    bias[j] = g.bias && c < g.N ? *(const f32x4u*)(g.bias + c) : (f32x4){0.f, 0.f, 0.f, 0.f};
+  }
+  constexpr int MTS = BN == 128 ? BM * MT_MAX : 1;
+  __shared__ float ms[MTS];                    // moment tensors of the tile's samples
+  const int smp0 = g.y ? m0 / g.rps : 0;
+  if (BN == 128 && g.y) {
+    const int n = ((min(m0 + BM, g.M) - 1) / g.rps - smp0 + 1) * g.nk;
+    for (int q = threadIdx.x; q < n; q += NT) ms[q] = g.mten[(long)smp0 * g.nk + q];
+  }
+#pragma unroll
+  for (int s = 0; s < NS - 1; ++s)
+    if (s < nk) load(s);
   for (int s = 0; s < nk; ++s) {
-    load(s + NS - 1);
-    asm volatile("s_waitcnt vmcnt(%0)\n\ts_barrier" ::"n"((NS - 1) * (OA::N + OB::N)) : "memory");
-    const uint16_t *pa = As[s % NS], *pb = Bs[s % NS];
+    if (s + NS - 1 < nk) {
+      load(s + NS - 1);
+      asm volatile("s_waitcnt vmcnt(%0)\n\ts_barrier" ::"n"((NS - 1) * (OA::N + OB::N)) : "memory");
+    } else {
+      asm volatile("s_waitcnt vmcnt(0)\n\ts_barrier" ::: "memory");
+    }
+    const uint16_t *pa = As + s % NS * (BM * BK), *pb = Bs + s % NS * (BN * BK);
 #pragma unroll
     for (int kk = 0; kk < BK; kk += 32) {
       bf16x8 a[FM], b[FN];
@@ -191,65 +257,164 @@ __global__ __launch_bounds__(64 * WM * WN) void gemm_bf16_kernel(GemmArgs g)
           for (int i = 0; i < FM; ++i)
             acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(b[j], a[i], acc[i][j], 0, 0, 0);
         }
+      if (TA && !TB && cs) {
+#pragma unroll
+        for (int j = 0; j < FN; ++j)
+          if (j < nj) sums[j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(b[j], ones, sums[j], 0, 0, 0);
+      }
     }
     // the stage is read before it is loaded again
     asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
   }
 
+  // (every load has landed and been read: the stages' LDS is free)
   // D layout of a 16x16 MFMA tile: lane l holds rows (here columns of C)
   // 4*(l/16)+e, column (row of C) l%16
+  if (TA && !TB && cs && (lane & 15) == 0) {
+    float* o = g.work ? g.work + (long)g.S * g.M * g.N + (long)tz * g.N : g.csum;
+#pragma unroll
+    for (int j = 0; j < FN; ++j) {
+      const int c = n0 + wn + 16 * j + 4 * (lane >> 4);
+      if (c < g.N) *(f32x4u*)(o + c) = sums[j];
+    }
+  }
+  // bf16 rows leave through the wave's own LDS, so that a store writes whole
+  // 128-byte lines and not 32 bytes of each of 16 rows
+  constexpr int WR = BM / WM, WC = BN / WN, WS = WC + 8;
+  static_assert(WM * WN * WR * WS == ROWS, "");
+  uint16_t* const st = sm + w * WR * WS;
+  constexpr int CH = WC / 8, NQ = WR * CH / 64;  // 16-byte pieces of a row, of a lane
+  static_assert(WR * CH % 64 == 0, "");
+  u16x8 keep[NQ];
+  float* const ct = (float*)sm;                // the block's rows for the contraction
+  const bool staged = g.C16 && g.vec16 && !g.work;
+  const bool masked = staged && g.epi == EPI_MASK;
+  if (masked) {
+#pragma unroll
+    for (int i = 0; i < NQ; ++i) {
+      const int q = i * 64 + lane, r = min(m0 + wm + q / CH, g.M - 1);
+      const int c = min(n0 + wn + q % CH * 8, g.N - 8);
+      keep[i] = *(const u16x8*)(g.mask + (long)r * g.ldm + c);
+    }
+  }
 #pragma unroll
   for (int j = 0; j < FN; ++j) {
-    const int c = n0 + wn + 16 * j + 4 * (lane >> 4);
+    const int cw = 16 * j + 4 * (lane >> 4), c = n0 + wn + cw;
     if (c >= g.N) continue;          // N is a multiple of 8: all four or none
-    f32x4 bias = {0.f, 0.f, 0.f, 0.f};
-    if (g.bias && !g.work) bias = *(const f32x4u*)(g.bias + c);
 #pragma unroll
     for (int i = 0; i < FM; ++i) {
-      const int r = m0 + wm + 16 * i + (lane & 15);
+      const int rw = 16 * i + (lane & 15), r = m0 + wm + rw;
       if (r >= g.M) continue;
       f32x4 v = acc[i][j];
       if (g.work) {
-        *(f32x4u*)(g.work + ((long)blockIdx.z * g.M + r) * g.N + c) = v;
+        *(f32x4u*)(g.work + ((long)tz * g.M + r) * g.N + c) = v;
         continue;
       }
-      if (g.bias) v = v + bias;
+      if (g.bias) v = v + bias[j];
+      if (BN == 128 && g.y) {
+        *(f32x4*)(ct + (wm + rw) * g.N + c) = v;
+        continue;
+      }
       if (g.epi == EPI_RELU) {
 #pragma unroll
         for (int e = 0; e < 4; ++e) v[e] = v[e] > 0.f ? v[e] : 0.f;
       }
-      if (g.epi == EPI_MASK) {
-        u16x4 h;
+      if (g.epi == EPI_MASK && (!staged || g.C32)) {
         const uint16_t* q = g.mask + (long)r * g.ldm + c;
-        if (g.vec16) h = *(const u16x4*)q;
-        else
-          for (int e = 0; e < 4; ++e) h[e] = q[e];
 #pragma unroll
-        for (int e = 0; e < 4; ++e) v[e] = bf_pos(h[e]) ? v[e] : 0.f;
+        for (int e = 0; e < 4; ++e) v[e] = bf_pos(q[e]) ? v[e] : 0.f;
       }
       if (g.C32) *(f32x4u*)(g.C32 + (long)r * g.ldc32 + c) = v;
       if (g.C16) {
         u16x4 h;
 #pragma unroll
         for (int e = 0; e < 4; ++e) h[e] = f2bf(v[e]);
-        uint16_t* q = g.C16 + (long)r * g.ldc16 + c;
-        if (g.vec16) *(u16x4*)q = h;
-        else
+        if (staged) {
+          *(u16x4*)(st + rw * WS + cw) = h;
+        } else {
+          uint16_t* q = g.C16 + (long)r * g.ldc16 + c;
           for (int e = 0; e < 4; ++e) q[e] = h[e];
+        }
       }
+    }
+  }
+  if (staged) {
+#pragma unroll
+    for (int i = 0; i < NQ; ++i) {
+      const int q = i * 64 + lane, rw = q / CH, r = m0 + wm + rw, c = n0 + wn + q % CH * 8;
+      u16x8 h = *(const u16x8*)(st + rw * WS + q % CH * 8);
+      if (masked) {
+#pragma unroll
+        for (int e = 0; e < 8; ++e) h[e] = bf_pos(keep[i][e]) ? h[e] : (uint16_t)0;
+      }
+      if (r < g.M && c < g.N) *(u16x8*)(g.C16 + (long)r * g.ldc16 + c) = h;
+    }
+  }
+  if (BN == 128 && g.y) {
+    __syncthreads();
+    const int rows = min(BM, g.M - m0), n4 = g.N / 4, no = g.N / g.nk;
+    for (int q = threadIdx.x; q < rows * n4; q += NT) {
+      const int r = q / n4, c = (q - r * n4) * 4;
+      *(f32x4u*)(g.C32 + (long)(m0 + r) * g.ldc32 + c) = *(const f32x4*)(ct + r * g.N + c);
+    }
+    for (int q = threadIdx.x; q < rows * no; q += NT) {
+      const int r = q / no, o = q - r * no, t = o / g.nc, c = o - t * g.nc;
+      const float* m = ms + ((m0 + r) / g.rps - smp0) * g.nk;
+      const float* a = ct + r * g.N + t * g.nk * g.nc + c;
+      float v = m[0] * a[0];
+      for (int k = 1; k < g.nk; ++k) v = v + m[k] * a[k * g.nc];
+      g.y[(long)(m0 + r) * no + o] = v;
     }
   }
 }
 
-// out[r][c] = sum over s of work[s][r][c], s in increasing order (deterministic)
-__global__ void splitk_reduce_kernel(int S, int M, int N, const float* work, float* out, long ldo)
+// out[r][c] = sum over s of work[s][r][c], and csum[c] the same of the partials
+// [S][N] behind them.  G threads share an output's partials, every G-th each,
+// and a tree over them closes it: the order is fixed (deterministic), and a sum
+// of 128 or 256 partials is no serial chain of loads.  A thread holds E
+// neighbouring outputs, E a divisor of N.  128 partials of 128 x 72 values 31 us
+// and 256 of 512 values 60 us one thread an output.
+template <int E>
+__global__ __launch_bounds__(256) void splitk_reduce_kernel(int S, int M, int N, int G,
+                                                           const float* work, float* out,
+                                                           long ldo, float* csum)
 {
-  const long i = (long)blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= (long)M * N) return;
-  const long r = i / N, c = i % N;
-  float s = 0.f;
-  for (int z = 0; z < S; ++z) s = s + work[(long)z * M * N + i];
-  out[r * ldo + c] = s;
+  typedef float vec __attribute__((ext_vector_type(E)));
+  typedef float vecu __attribute__((ext_vector_type(E), aligned(4)));
+  __shared__ vec part[256];
+  const int L = 256 / G, l = threadIdx.x % L, zg = threadIdx.x / L;
+  const long n = (long)M * N, i = ((long)blockIdx.x * L + l) * E;
+  const long end = n + (csum ? N : 0);
+  vec s = (vec)(0.f);
+  if (i < end) {
+    const float* p = i < n ? work + i : work + S * n + (i - n);
+    const long step = i < n ? n : N;
+#pragma unroll 4
+    for (int z = zg; z < S; z += G) s = s + *(const vecu*)(p + z * step);
+  }
+  part[threadIdx.x] = s;
+  __syncthreads();
+  for (int h = G / 2; h > 0; h >>= 1) {
+    if (zg < h) part[threadIdx.x] = part[threadIdx.x] + part[threadIdx.x + h * L];
+    __syncthreads();
+  }
+  if (zg || i >= end) return;
+  float* o = i < n ? out + i / N * ldo + i % N : csum + (i - n);
+  *(vecu*)o = part[l];
+}
+
+static void launch_reduce(hipStream_t st, int S, int M, int N, const float* work, float* out,
+                          long ldo, float* csum)
+{
+  int G = 1;
+  while (G < 32 && G * 4 <= S) G *= 2;
+  const long n = (long)M * N + (csum ? N : 0), L = 256 / G;
+  if (N % 4 == 0)
+    hipLaunchKernelGGL(splitk_reduce_kernel<4>, dim3((unsigned)((n / 4 + L - 1) / L)), dim3(256),
+                       0, st, S, M, N, G, work, out, ldo, csum);
+  else
+    hipLaunchKernelGGL(splitk_reduce_kernel<1>, dim3((unsigned)((n + L - 1) / L)), dim3(256), 0,
+                       st, S, M, N, G, work, out, ldo, csum);
 }
 
 // partial column sums of a bf16 matrix: block (x, y) sums rows of split y for
@@ -297,12 +462,10 @@ __global__ __launch_bounds__(256) void loss_grad_kernel(long n, const float* Y, 
 }
 
 // Adam on FP32 master values; w16 (optional) receives the bf16 copy
-__global__ void adam_kernel(long n, float* w, float* m, float* v, const float* g, uint16_t* w16,
-                            float lr, float b1, float b2, float c1, float c2, float bc1, float bc2,
-                            float eps)
+__device__ __forceinline__ void adam_one(long i, float* w, float* m, float* v, const float* g,
+                                         uint16_t* w16, float lr, float b1, float b2, float c1,
+                                         float c2, float bc1, float bc2, float eps)
 {
-  const long i = (long)blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= n) return;
   const float gi = g[i];
   const float mi = b1 * m[i] + c1 * gi;
   const float vi = b2 * v[i] + c2 * (gi * gi);
@@ -314,55 +477,101 @@ __global__ void adam_kernel(long n, float* w, float* m, float* v, const float* g
   if (w16) w16[i] = f2bf(wi);
 }
 
-// moment-tensor contraction of basis waveforms, one block per sample:
-// y[b][t][c] = sum_k m[b][k] g[b][t][k][c] (k in increasing order)
-constexpr int MT_MAX = 8;
-
-__global__ __launch_bounds__(256) void mt_contract_kernel(int nt, int nc, int nk, const float* m,
-                                                         const float* g, float* y)
+__global__ void adam_kernel(long n, float* w, float* m, float* v, const float* g, uint16_t* w16,
+                            float lr, float b1, float b2, float c1, float c2, float bc1, float bc2,
+                            float eps)
 {
-  const int b = blockIdx.x;
-  float mk[MT_MAX];
-  for (int k = 0; k < nk; ++k) mk[k] = m[b * nk + k];
-  const long n = (long)nt * nc;
-  const float* gb = g + (long)b * n * nk;
-  for (long e = threadIdx.x; e < n; e += 256) {
-    const long t = e / nc, c = e - t * nc;
-    const float* q = gb + t * nk * nc + c;
+  const long i = (long)blockIdx.x * blockDim.x + threadIdx.x;
+  if (i >= n) return;
+  adam_one(i, w, m, v, g, w16, lr, b1, b2, c1, c2, bc1, bc2, eps);
+}
+
+// the same for several tensors in one launch, 1024 values a block: a network's
+// 16 launches of 2 to 12 us, most of them a few blocks
+constexpr int ADAM_MAX = 32;
+struct AdamList {
+  int count;
+  unsigned start[ADAM_MAX + 1];   // first block of each tensor
+  long n[ADAM_MAX];
+  float *w[ADAM_MAX], *m[ADAM_MAX], *v[ADAM_MAX];
+  const float* g[ADAM_MAX];
+  uint16_t* w16[ADAM_MAX];
+};
+
+__global__ __launch_bounds__(256) void adam_multi_kernel(AdamList a, float lr, float b1, float b2,
+                                                        float c1, float c2, float bc1, float bc2,
+                                                        float eps)
+{
+  int q = 0;
+  while (q + 1 < a.count && blockIdx.x >= a.start[q + 1]) ++q;
+  const long i0 = (long)(blockIdx.x - a.start[q]) * 1024 + threadIdx.x;
+#pragma unroll
+  for (int e = 0; e < 4; ++e)
+    if (i0 + e * 256 < a.n[q])
+      adam_one(i0 + e * 256, a.w[q], a.m[q], a.v[q], a.g[q], a.w16[q], lr, b1, b2, c1, c2, bc1,
+               bc2, eps);
+}
+
+// moment-tensor contraction of basis waveforms, one block per sample:
+// y[b][t][c] = sum_k m[b][k] g[b][t][k][c] (k in increasing order).  NK terms,
+// known when compiled: their loads leave together, not one latency after
+// another, and 32-bit indices, for which a division is a few instructions
+// (the host sees to it that they suffice).
+template <int NK>
+__global__ __launch_bounds__(256) void mt_contract_kernel(unsigned nt, unsigned nc,
+                                                         const float* __restrict__ m,
+                                                         const float* __restrict__ g,
+                                                         float* __restrict__ y)
+{
+  const long b = blockIdx.x;
+  float mk[NK];
+#pragma unroll
+  for (int k = 0; k < NK; ++k) mk[k] = m[b * NK + k];
+  const unsigned n = nt * nc;
+  const float* gb = g + b * n * NK;
+#pragma unroll 2
+  for (unsigned e = threadIdx.x; e < n; e += 256) {
+    const unsigned t = e / nc;
+    const float* q = gb + (t * (NK - 1) * nc + e);
     float v = mk[0] * q[0];
-    for (int k = 1; k < nk; ++k) v = v + mk[k] * q[(long)k * nc];
-    y[(long)b * n + e] = v;
+#pragma unroll
+    for (int k = 1; k < NK; ++k) v = v + mk[k] * q[k * nc];
+    y[b * n + e] = v;
   }
 }
 
 // the contraction fused with the per-sample relative misfit and its gradient
 // with respect to the basis waveforms: dg[b][t][k][c] = bf16(m[b][k] dy[b][t][c]),
 // dy = 2 (y - T) / (nsamp (tn2[b] + eps))
-__global__ __launch_bounds__(256) void mt_loss_grad_kernel(int nt, int nc, int nk, const float* m,
-                                                          const float* g, const float* T,
-                                                          const float* tn2, float eps, int nsamp,
-                                                          uint16_t* dg, float* loss)
+template <int NK>
+__global__ __launch_bounds__(256) void mt_loss_grad_kernel(
+    unsigned nt, unsigned nc, const float* __restrict__ m, const float* __restrict__ g,
+    const float* __restrict__ T, const float* __restrict__ tn2, float eps, int nsamp,
+    uint16_t* __restrict__ dg, float* __restrict__ loss)
 {
   __shared__ float red[256];
-  const int b = blockIdx.x;
-  float mk[MT_MAX];
-  for (int k = 0; k < nk; ++k) mk[k] = m[b * nk + k];
+  const long b = blockIdx.x;
+  float mk[NK];
+#pragma unroll
+  for (int k = 0; k < NK; ++k) mk[k] = m[b * NK + k];
   const float den = tn2[b] + eps;
   const float scale = 2.0f / ((float)nsamp * den);
-  const long n = (long)nt * nc;
-  const float* gb = g + (long)b * n * nk;
-  uint16_t* db = dg ? dg + (long)b * n * nk : nullptr;
+  const unsigned n = nt * nc;
+  const float* gb = g + b * n * NK;
+  uint16_t* db = dg ? dg + b * n * NK : nullptr;
   float s = 0.f;
-  for (long e = threadIdx.x; e < n; e += 256) {
-    const long t = e / nc, c = e - t * nc;
-    const long o = t * nk * nc + c;
+#pragma unroll 2
+  for (unsigned e = threadIdx.x; e < n; e += 256) {
+    const unsigned o = e / nc * (NK - 1) * nc + e;
     float v = mk[0] * gb[o];
-    for (int k = 1; k < nk; ++k) v = v + mk[k] * gb[o + (long)k * nc];
-    const float d = v - T[(long)b * n + e];
+#pragma unroll
+    for (int k = 1; k < NK; ++k) v = v + mk[k] * gb[o + k * nc];
+    const float d = v - T[b * n + e];
     s = s + d * d;
     if (db) {
       const float dy = d * scale;
-      for (int k = 0; k < nk; ++k) db[o + (long)k * nc] = f2bf(mk[k] * dy);
+#pragma unroll
+      for (int k = 0; k < NK; ++k) db[o + k * nc] = f2bf(mk[k] * dy);
     }
   }
   red[threadIdx.x] = s;
@@ -373,6 +582,19 @@ __global__ __launch_bounds__(256) void mt_loss_grad_kernel(int nt, int nc, int n
   }
   if (threadIdx.x == 0) loss[b] = red[0] / den;
 }
+
+// a kernel of the number of terms
+#define CGFDS_TERMS(nk, F) \
+  switch (nk) {            \
+  case 1: F(1); break;     \
+  case 2: F(2); break;     \
+  case 3: F(3); break;     \
+  case 4: F(4); break;     \
+  case 5: F(5); break;     \
+  case 6: F(6); break;     \
+  case 7: F(7); break;     \
+  default: F(8); break;    \
+  }
 
 __global__ void to_bf16_kernel(long n, const float* src, uint16_t* dst)
 {
@@ -395,73 +617,141 @@ static int launch_check(const char* what)
 
 using namespace cgfds;
 
-extern "C" int cgfds_gemm_bf16(int M, int N, int K, const void* A, long lda, int transA,
-                               const void* B, long ldb, int transB, const float* bias,
-                               int epilogue, const void* mask, long ldm, float* C32, long ldc32,
-                               void* C16, long ldc16, int splitk, float* work, void* stream)
+// what the products have in common: the checks, the split of the contraction,
+// the tile, the order of the blocks, the launches
+static int gemm_launch(const char* name, GemmArgs g, int transA, int transB, int splitk,
+                       float* work, hipStream_t st)
 {
-  if (M <= 0 || N <= 0 || K <= 0 || !A || !B || (!C32 && !C16))
-    return sfail(CGFDH_EINVAL, "cgfds_gemm_bf16: empty shape or null operand");
-  if (M % 8 || N % 8 || K % 8 || lda % 8 || ldb % 8 || !al16(A) || !al16(B))
-    return sfail(CGFDH_EINVAL,
-                 "cgfds_gemm_bf16: M, N, K and the A/B leading dimensions must be multiples "
-                 "of 8 and A, B 16-byte aligned");
-  if (lda < (transA ? M : K) || ldb < (transB ? K : N) || (C32 && ldc32 < N) ||
-      (C16 && ldc16 < N))
-    return sfail(CGFDH_EINVAL, "cgfds_gemm_bf16: leading dimension below the row length");
-  if (epilogue < EPI_NONE || epilogue > EPI_MASK || (epilogue == EPI_MASK && (!mask || ldm < N)))
-    return sfail(CGFDH_EINVAL, "cgfds_gemm_bf16: bad epilogue or missing mask");
-  if (splitk < 1 || splitk > 1024)
-    return sfail(CGFDH_EINVAL, "cgfds_gemm_bf16: splitk outside 1..1024");
-  int kchunk = ((K + splitk - 1) / splitk + 31) / 32 * 32;
-  int S = (K + kchunk - 1) / kchunk;
-  if (S > 1 && (!work || !C32 || C16 || bias || epilogue != EPI_NONE))
-    return sfail(CGFDH_EINVAL,
-                 "cgfds_gemm_bf16: split-K needs a work buffer, FP32 output and no epilogue");
-  auto al8 = [](const void* p, long ld) { return !p || (((uintptr_t)p & 7u) == 0 && ld % 4 == 0); };
-  GemmArgs g{M, N, K, (const uint16_t*)A, lda, (const uint16_t*)B, ldb, bias, epilogue,
-             (const uint16_t*)mask, ldm, C32, ldc32, (uint16_t*)C16, ldc16, kchunk,
-             S > 1 ? work : nullptr, al8(mask, ldm) && al8(C16, ldc16)};
-  hipStream_t st = (hipStream_t)stream;
-  if ((N + 63) / 64 > 65535)
-    return sfail(CGFDH_EINVAL, "cgfds_gemm_bf16: N above 65535*64 columns");
+  auto bad = [&](const char* why) {
+    char buf[256];
+    snprintf(buf, sizeof buf, "%s: %s", name, why);
+    return sfail(CGFDH_EINVAL, buf);
+  };
+  const int M = g.M, N = g.N, K = g.K;
+  if (M <= 0 || N <= 0 || K <= 0 || !g.A || !g.B || (!g.C32 && !g.C16))
+    return bad("empty shape or null operand");
+  if (M % 8 || N % 8 || K % 8 || g.lda % 8 || g.ldb % 8 || !al16(g.A) || !al16(g.B))
+    return bad("M, N, K and the A/B leading dimensions must be multiples "
+               "of 8 and A, B 16-byte aligned");
+  if (g.lda < (transA ? M : K) || g.ldb < (transB ? K : N) || (g.C32 && g.ldc32 < N) ||
+      (g.C16 && g.ldc16 < N))
+    return bad("leading dimension below the row length");
+  if (g.epi < EPI_NONE || g.epi > EPI_MASK || (g.epi == EPI_MASK && (!g.mask || g.ldm < N)))
+    return bad("bad epilogue or missing mask");
+  if (splitk < 1 || splitk > 1024) return bad("splitk outside 1..1024");
+  if ((N + 63) / 64 > 65535) return bad("N above 65535*64 columns");
+  g.kchunk = ((K + splitk - 1) / splitk + 31) / 32 * 32;
+  const int S = g.S = (K + g.kchunk - 1) / g.kchunk;
+  if (S > 1 && (!work || !g.C32 || g.C16 || g.bias || g.epi != EPI_NONE))
+    return bad("split-K needs a work buffer, FP32 output and no epilogue");
+  g.work = S > 1 ? work : nullptr;
+  auto vec = [](const void* p, long ld) { return !p || (al16(p) && ld % 8 == 0); };
+  g.vec16 = vec(g.mask, g.ldm) && vec(g.C16, g.ldc16);
   const int form = (transA ? 2 : 0) + (transB ? 1 : 0);
-  // row tiles on x (up to 2^31 - 1 blocks), column tiles on y
-  auto launch = [&](auto bm, auto bn, auto bk, auto ns, auto wm, auto wn) {
+  // Whole groups of blocks go to an XCD where there are enough of them: the
+  // tiles of one range of the contraction read the same rows of A and B, the
+  // column tiles of a row tile the same rows of A.
+  auto shape = [&](int BM, int BN) {
+    g.mt = (M + BM - 1) / BM;
+    g.nt = (N + BN - 1) / BN;
+    g.order = S >= 8 ? ORD_SPLIT : (S == 1 && g.nt > 1 && g.mt >= 64 ? ORD_ROWS : ORD_PLAIN);
+    if (g.order == ORD_ROWS) return (long)((g.mt + 7) / 8 * 8) * g.nt;
+    return (long)g.mt * g.nt * (g.order == ORD_SPLIT ? (S + 7) / 8 * 8 : S);
+  };
+  long blocks = 0;
+  auto launch = [&](auto bm, auto bn, auto bk, auto ns, auto wm) {
     constexpr int BM = decltype(bm)::value, BN = decltype(bn)::value, BK = decltype(bk)::value,
-                  NS = decltype(ns)::value, WM = decltype(wm)::value, WN = decltype(wn)::value;
-    const dim3 grid((M + BM - 1) / BM, (N + BN - 1) / BN, S), blk(64 * WM * WN);
+                  NS = decltype(ns)::value, WM = decltype(wm)::value;
+    blocks = shape(BM, BN);
+    if (blocks > 0x7fffffffl) return;
+    const dim3 grid((unsigned)blocks), blk(128 * WM);
     switch (form) {
-    case 0: hipLaunchKernelGGL((gemm_bf16_kernel<0, 0, BM, BN, BK, NS, WM, WN>), grid, blk, 0, st, g); break;
-    case 1: hipLaunchKernelGGL((gemm_bf16_kernel<0, 1, BM, BN, BK, NS, WM, WN>), grid, blk, 0, st, g); break;
-    case 2: hipLaunchKernelGGL((gemm_bf16_kernel<1, 0, BM, BN, BK, NS, WM, WN>), grid, blk, 0, st, g); break;
-    default: hipLaunchKernelGGL((gemm_bf16_kernel<1, 1, BM, BN, BK, NS, WM, WN>), grid, blk, 0, st, g); break;
+    case 0: hipLaunchKernelGGL((gemm_bf16_kernel<0, 0, BM, BN, BK, NS, WM, 2>), grid, blk, 0, st, g); break;
+    case 1: hipLaunchKernelGGL((gemm_bf16_kernel<0, 1, BM, BN, BK, NS, WM, 2>), grid, blk, 0, st, g); break;
+    case 2: hipLaunchKernelGGL((gemm_bf16_kernel<1, 0, BM, BN, BK, NS, WM, 2>), grid, blk, 0, st, g); break;
+    default: hipLaunchKernelGGL((gemm_bf16_kernel<1, 1, BM, BN, BK, NS, WM, 2>), grid, blk, 0, st, g); break;
     }
   };
 #define CGFDS_I(n) std::integral_constant<int, n>{}
   // The largest tile that still leaves a block for each of the 256 compute
   // units: fewer bytes through LDS a product.  us, 128 x 128 and 64 x 64:
-  // 2048 x 4096 x 512 (512 large tiles) 23, 31; 2048 x 512 x 512 (64) 16, 9.
+  // 2048 x 4096 x 512 (512 large tiles) 22, 31; 2048 x 512 x 512 (64) 13, 9.
+  // Short contractions are bound by the latency of a block's loads and stores,
+  // so the large tile has 8 waves: 1048576 x 512 x 128 493 us (2.7 TB/s), with 4
+  // waves 595, in 64 x 128 tiles 582; 16384 x 4096 x 512 130, 144, 154.
   // Where even 64 x 64 leaves units idle the contraction is a serial chain, so
   // fewer, deeper stages and twice the tiles: 64 x 512 x 4096 28, 37; 512 x 512
-  // x 4096 34, 51; level with 64 x 64 at K = 512 and below.
+  // x 4096 29, 51; level with 64 x 64 at K = 512 and below.
   const long big = (long)((M + 127) / 128) * ((N + 127) / 128) * S;
   const long mid = (long)((M + 63) / 64) * ((N + 63) / 64) * S;
-  if (big >= 256)
-    launch(CGFDS_I(128), CGFDS_I(128), CGFDS_I(64), CGFDS_I(2), CGFDS_I(2), CGFDS_I(2));
-  else if (mid >= 256)
-    launch(CGFDS_I(64), CGFDS_I(64), CGFDS_I(64), CGFDS_I(3), CGFDS_I(2), CGFDS_I(2));
-  else
-    launch(CGFDS_I(64), CGFDS_I(32), CGFDS_I(128), CGFDS_I(4), CGFDS_I(2), CGFDS_I(2));
+  if (big >= 256) {
+    launch(CGFDS_I(128), CGFDS_I(128), CGFDS_I(64), CGFDS_I(2), CGFDS_I(4));
+  } else if (g.y) {
+    // the contraction needs whole rows in a block
+    blocks = shape(64, 128);
+    hipLaunchKernelGGL((gemm_bf16_kernel<0, 0, 64, 128, 64, 3, 2, 2>), dim3((unsigned)blocks),
+                       dim3(256), 0, st, g);
+  } else if (mid >= 256) {
+    launch(CGFDS_I(64), CGFDS_I(64), CGFDS_I(64), CGFDS_I(3), CGFDS_I(2));
+  } else {
+    launch(CGFDS_I(64), CGFDS_I(32), CGFDS_I(128), CGFDS_I(4), CGFDS_I(2));
+  }
 #undef CGFDS_I
-  if (int rc = launch_check("cgfds_gemm_bf16")) return rc;
+  if (blocks > 0x7fffffffl) return bad("more than 2^31 - 1 tiles");
+  if (int rc = launch_check(name)) return rc;
   if (S > 1) {
-    long n = (long)M * N;
-    hipLaunchKernelGGL(splitk_reduce_kernel, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, st,
-                       S, M, N, (const float*)work, C32, ldc32);
-    return launch_check("cgfds_gemm_bf16 (split-K reduce)");
+    launch_reduce(st, S, M, N, work, g.C32, g.ldc32, g.csum);
+    return launch_check(name);
   }
   return 0;
+}
+
+extern "C" int cgfds_gemm_bf16(int M, int N, int K, const void* A, long lda, int transA,
+                               const void* B, long ldb, int transB, const float* bias,
+                               int epilogue, const void* mask, long ldm, float* C32, long ldc32,
+                               void* C16, long ldc16, int splitk, float* work, void* stream)
+{
+  GemmArgs g = {};
+  g.M = M; g.N = N; g.K = K;
+  g.A = (const uint16_t*)A; g.lda = lda;
+  g.B = (const uint16_t*)B; g.ldb = ldb;
+  g.bias = bias; g.epi = epilogue;
+  g.mask = (const uint16_t*)mask; g.ldm = ldm;
+  g.C32 = C32; g.ldc32 = ldc32;
+  g.C16 = (uint16_t*)C16; g.ldc16 = ldc16;
+  return gemm_launch("cgfds_gemm_bf16", g, transA, transB, splitk, work, (hipStream_t)stream);
+}
+
+extern "C" int cgfds_gemm_bf16_colsum(int M, int N, int K, const void* A, long lda, const void* G,
+                                      long ldg, float* C32, long ldc32, float* csum, int splitk,
+                                      float* work, void* stream)
+{
+  if (!C32 || !csum) return sfail(CGFDH_EINVAL, "cgfds_gemm_bf16_colsum: null output");
+  GemmArgs g = {};
+  g.M = M; g.N = N; g.K = K;
+  g.A = (const uint16_t*)A; g.lda = lda;
+  g.B = (const uint16_t*)G; g.ldb = ldg;
+  g.C32 = C32; g.ldc32 = ldc32;
+  g.csum = csum;
+  return gemm_launch("cgfds_gemm_bf16_colsum", g, 1, 0, splitk, work, (hipStream_t)stream);
+}
+
+extern "C" int cgfds_gemm_bf16_mt(int M, int N, int K, const void* A, long lda, const void* B,
+                                  long ldb, const float* bias, float* C32, long ldc32, int nk,
+                                  int nc, int rps, const float* m, float* y, void* stream)
+{
+  if (!C32 || !m || !y || nk < 1 || nk > MT_MAX || nc < 1 || rps < 1 || N > 128 ||
+      (long)N % ((long)nk * nc))
+    return sfail(CGFDH_EINVAL, "cgfds_gemm_bf16_mt: bad argument (N must be a multiple of "
+                               "nk * nc of at most 128, nk 1..8)");
+  GemmArgs g = {};
+  g.M = M; g.N = N; g.K = K;
+  g.A = (const uint16_t*)A; g.lda = lda;
+  g.B = (const uint16_t*)B; g.ldb = ldb;
+  g.bias = bias;
+  g.C32 = C32; g.ldc32 = ldc32;
+  g.mten = m; g.y = y; g.nk = nk; g.nc = nc; g.rps = rps;
+  return gemm_launch("cgfds_gemm_bf16_mt", g, 0, 0, 1, nullptr, (hipStream_t)stream);
 }
 
 extern "C" int cgfds_colsum_bf16(int M, int N, const void* G, long ldg, float* out, int splits,
@@ -473,8 +763,7 @@ extern "C" int cgfds_colsum_bf16(int M, int N, const void* G, long ldg, float* o
   hipLaunchKernelGGL(colsum_bf16_kernel, dim3((N + 63) / 64, splits), dim3(256), 0, st, M, N,
                      (const uint16_t*)G, ldg, splits, work);
   if (int rc = launch_check("cgfds_colsum_bf16")) return rc;
-  hipLaunchKernelGGL(splitk_reduce_kernel, dim3((N + 255) / 256), dim3(256), 0, st, splits, 1, N,
-                     (const float*)work, out, (long)N);
+  launch_reduce(st, splits, 1, N, work, out, N, nullptr);
   return launch_check("cgfds_colsum_bf16 (reduce)");
 }
 
@@ -500,13 +789,46 @@ extern "C" int cgfds_adam(long n, float* w, float* m, float* v, const float* g, 
   return launch_check("cgfds_adam");
 }
 
+extern "C" int cgfds_adam_multi(int count, const long* n, float* const* w, float* const* m,
+                                float* const* v, const float* const* g, void* const* w16, float lr,
+                                float b1, float b2, float c1, float c2, float bc1, float bc2,
+                                float eps, void* stream)
+{
+  if (count <= 0 || !n || !w || !m || !v || !g || !w16)
+    return sfail(CGFDH_EINVAL, "cgfds_adam_multi: bad argument");
+  for (int q = 0; q < count; ++q)
+    if (n[q] <= 0 || n[q] > 1l << 40 || !w[q] || !m[q] || !v[q] || !g[q])
+      return sfail(CGFDH_EINVAL, "cgfds_adam_multi: bad tensor");
+  for (int q0 = 0; q0 < count; q0 += ADAM_MAX) {
+    AdamList a = {};
+    a.count = std::min(ADAM_MAX, count - q0);
+    for (int q = 0; q < a.count; ++q) {
+      a.n[q] = n[q0 + q];
+      a.w[q] = w[q0 + q]; a.m[q] = m[q0 + q]; a.v[q] = v[q0 + q]; a.g[q] = g[q0 + q];
+      a.w16[q] = (uint16_t*)w16[q0 + q];
+      const long end = a.start[q] + (a.n[q] + 1023) / 1024;
+      if (end > 0x7fffffffl) return sfail(CGFDH_EINVAL, "cgfds_adam_multi: too many values");
+      a.start[q + 1] = (unsigned)end;
+    }
+    hipLaunchKernelGGL(adam_multi_kernel, dim3(a.start[a.count]), dim3(256), 0,
+                       (hipStream_t)stream, a, lr, b1, b2, c1, c2, bc1, bc2, eps);
+    if (int rc = launch_check("cgfds_adam_multi")) return rc;
+  }
+  return 0;
+}
+
 extern "C" int cgfds_mt_contract(int nsamp, int nt, int nc, int nk, const float* m,
                                  const float* g, float* y, void* stream)
 {
   if (nsamp <= 0 || nt <= 0 || nc <= 0 || nk < 1 || nk > MT_MAX || !m || !g || !y)
     return sfail(CGFDH_EINVAL, "cgfds_mt_contract: bad argument (nk must be 1..8)");
-  hipLaunchKernelGGL(mt_contract_kernel, dim3(nsamp), dim3(256), 0, (hipStream_t)stream, nt, nc,
-                     nk, m, g, y);
+  if ((double)nt * nc * nk > 2147483647.0)
+    return sfail(CGFDH_EINVAL, "cgfds_mt_contract: more than 2^31 - 1 values a sample");
+#define CGFDS_F(n)                                                                        \
+  hipLaunchKernelGGL(mt_contract_kernel<n>, dim3(nsamp), dim3(256), 0, (hipStream_t)stream, \
+                     (unsigned)nt, (unsigned)nc, m, g, y)
+  CGFDS_TERMS(nk, CGFDS_F)
+#undef CGFDS_F
   return launch_check("cgfds_mt_contract");
 }
 
@@ -517,8 +839,14 @@ extern "C" int cgfds_mt_loss_grad(int nsamp, int nt, int nc, int nk, const float
   if (nsamp <= 0 || nt <= 0 || nc <= 0 || nk < 1 || nk > MT_MAX || !m || !g || !T || !tnorm2 ||
       !loss)
     return sfail(CGFDH_EINVAL, "cgfds_mt_loss_grad: bad argument (nk must be 1..8)");
-  hipLaunchKernelGGL(mt_loss_grad_kernel, dim3(nsamp), dim3(256), 0, (hipStream_t)stream, nt, nc,
-                     nk, m, g, T, tnorm2, eps, nsamp, (uint16_t*)dg16, loss);
+  if ((double)nt * nc * nk > 2147483647.0)
+    return sfail(CGFDH_EINVAL, "cgfds_mt_loss_grad: more than 2^31 - 1 values a sample");
+#define CGFDS_F(n)                                                                         \
+  hipLaunchKernelGGL(mt_loss_grad_kernel<n>, dim3(nsamp), dim3(256), 0, (hipStream_t)stream, \
+                     (unsigned)nt, (unsigned)nc, m, g, T, tnorm2, eps, nsamp,              \
+                     (uint16_t*)dg16, loss)
+  CGFDS_TERMS(nk, CGFDS_F)
+#undef CGFDS_F
   return launch_check("cgfds_mt_loss_grad");
 }
 

@@ -80,6 +80,17 @@ def gemm(M, N, K, A, lda, transA, B, ldb, transB, bias=None, epi=EPI_NONE, mask=
                                 ldc16, splitk, _ptr(work), _stream()), "gemm_bf16")
 
 
+def gemm_colsum(M, N, K, A, lda, G, ldg, C32, csum, splitk, work):
+    check(lib().cgfds_gemm_bf16_colsum(M, N, K, _ptr(A), lda, _ptr(G), ldg, _ptr(C32), N,
+                                       _ptr(csum), splitk, _ptr(work), _stream()),
+          "gemm_bf16_colsum")
+
+
+def gemm_mt(M, N, K, A, B, bias, C32, nk, nc, rps, m, y):
+    check(lib().cgfds_gemm_bf16_mt(M, N, K, _ptr(A), K, _ptr(B), N, _ptr(bias), _ptr(C32), N, nk,
+                                   nc, rps, _ptr(m), _ptr(y), _stream()), "gemm_bf16_mt")
+
+
 def colsum(M, N, G, ldg, out, splits, work):
     check(lib().cgfds_colsum_bf16(M, N, _ptr(G), ldg, _ptr(out), splits, _ptr(work), _stream()),
           "colsum_bf16")
@@ -95,6 +106,16 @@ def adam(w, m, v, g, w16, lr, t, b1=0.9, b2=0.999, eps=1e-8):
     check(lib().cgfds_adam(w.numel(), _ptr(w), _ptr(m), _ptr(v), _ptr(g), _ptr(w16), lr, b1, b2,
                            1.0 - b1, 1.0 - b2, 1.0 - b1 ** t, 1.0 - b2 ** t, eps, _stream()),
           "adam")
+
+
+def adam_multi(tensors, lr, t, b1=0.9, b2=0.999, eps=1e-8):
+    """One Adam step on a list of (w, m, v, g, w16 or None)."""
+    k = len(tensors)
+    n = (C.c_long * k)(*[q[0].numel() for q in tensors])
+    cols = [(C.c_void_p * k)(*[None if q[j] is None else q[j].data_ptr() for q in tensors])
+            for j in range(5)]
+    check(lib().cgfds_adam_multi(k, n, *cols, lr, b1, b2, 1.0 - b1, 1.0 - b2, 1.0 - b1 ** t,
+                                 1.0 - b2 ** t, eps, _stream()), "adam_multi")
 
 
 def mt_contract(nsamp, nt, nc, nk, m, g, y):
@@ -183,7 +204,7 @@ class SurrogateNet:
         wk = 0
         for r, (k, n, _) in zip(rows, self.layers):
             s = _splitk(k, n, r)
-            wk = max(wk, s * k * n if s > 1 else 0, 256 * n)
+            wk = max(wk, s * (k + 1) * n if s > 1 else 0)
         work = torch.empty(wk, dtype=torch.float32, device=self.dev)
         x32 = torch.empty((nsamp, self.layers[0][0]), dtype=torch.float32, device=self.dev)
         loss = torch.empty(nsamp, dtype=torch.float32, device=self.dev)
@@ -214,9 +235,15 @@ class SurrogateNet:
         Returns the FP32 prediction (a view of an internal buffer, valid
         until the next call with the same nsamp): [rows_last, N_last], or
         [nsamp * nt, nc] after the moment-tensor contraction."""
-        torch = self.torch
         nsamp = nsamp or x.shape[0]
         b = self._buffers(nsamp)
+        self._layers(b, x, m, contract=True)
+        return b["yc"] if self.mt_terms else b["y"]
+
+    def _layers(self, b, x, m, contract):
+        """The layers into b["y"] and, with a moment-tensor output and
+        contract, b["yc"]."""
+        torch = self.torch
         self._set_m(b, m)
         if isinstance(x, np.ndarray):
             b["x32"].copy_(torch.from_numpy(np.ascontiguousarray(x, np.float32)))
@@ -225,17 +252,22 @@ class SurrogateNet:
         to_bf16(b["x32"], b["h"][0])
         rows = b["rows"]
         last = len(self.layers) - 1
+        nt, nc = self.out_shape if self.mt_terms else (0, 0)
         for li, (k, n, act) in enumerate(self.layers):
+            # whole rows of whole times that fit a tile are contracted where
+            # they are formed
+            if (li == last and contract and self.mt_terms and not act and n <= 128
+                    and n % (self.mt_terms * nc) == 0):
+                gemm_mt(rows[li], n, k, b["h"][li], self.w16[li], self.b32[li], b["y"],
+                        self.mt_terms, nc, nt * nc * self.mt_terms // n, b["m"], b["yc"])
+                return
             out16 = b["h"][li + 1] if li < last else None
             gemm(rows[li], n, k, b["h"][li], k, 0, self.w16[li], n, 0, bias=self.b32[li],
                  epi=EPI_RELU if act else EPI_NONE,
                  C32=b["y"] if li == last else None, ldc32=n,
                  C16=out16, ldc16=n)
-        if self.mt_terms:
-            nt, nc = self.out_shape
-            mt_contract(nsamp, nt, nc, self.mt_terms, b["m"], b["y"], b["yc"])
-            return b["yc"]
-        return b["y"]
+        if self.mt_terms and contract:
+            mt_contract(b["loss"].numel(), nt, nc, self.mt_terms, b["m"], b["y"], b["yc"])
 
     def backward(self, nsamp):
         """Gradients of every parameter from the bf16 output gradient already
@@ -247,11 +279,9 @@ class SurrogateNet:
             k, n, _ = self.layers[li]
             r = rows[li]
             g = b["g"][li]
-            # dW = H^T G  (K x N, reduction over the r rows)
-            s = _splitk(k, n, r)
-            gemm(k, n, r, b["h"][li], k, 1, g, n, 0, C32=self.gw[li], ldc32=n, splitk=s,
-                 work=work)
-            colsum(r, n, g, n, self.gb[li], min(256, max(1, r // 64)), work)
+            # dW = H^T G  (K x N, reduction over the r rows) and G's column sums
+            gemm_colsum(k, n, r, b["h"][li], k, g, n, self.gw[li], self.gb[li],
+                        _splitk(k, n, r), work)
             if li > 0:
                 # dH = G W^T, masked by the ReLU of the previous layer, to bf16
                 gemm(r, k, n, g, n, 0, self.w16[li], n, 1, epi=EPI_MASK, mask=b["h"][li], ldm=k,
@@ -259,14 +289,16 @@ class SurrogateNet:
 
     def adam_step(self, lr):
         self.t += 1
-        for li in range(len(self.layers)):
-            adam(self.w32[li], self.mw[li], self.vw[li], self.gw[li], self.w16[li], lr, self.t)
-            adam(self.b32[li], self.mb[li], self.vb[li], self.gb[li], None, lr, self.t)
+        adam_multi(list(zip(self.w32, self.mw, self.vw, self.gw, self.w16)) +
+                   [(w, m, v, g, None)
+                    for w, m, v, g in zip(self.b32, self.mb, self.vb, self.gb)], lr, self.t)
 
     def _loss(self, x, t, tn2, eps, m, grad):
         nsamp = x.shape[0]
-        y = self.forward(x, nsamp, m)
-        b = self._bufs[nsamp]
+        b = self._buffers(nsamp)
+        # the misfit kernel contracts the basis waveforms itself
+        self._layers(b, x, m, contract=False)
+        y = b["y"]
         g16 = b["g"][-1] if grad else None
         if self.mt_terms:
             nt, nc = self.out_shape

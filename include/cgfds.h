@@ -37,6 +37,21 @@ int cgfds_gemm_bf16(int M, int N, int K, const void *A, long lda, int transA, co
                     long ldm, float *C32, long ldc32, void *C16, long ldc16, int splitk,
                     float *work, void *stream);
 
+/* A weight gradient and its bias gradient from one reading of G: C32[M][N] =
+ * sum_k A[k][m] G[k][n] and csum[n] = sum_k G[k][n].  splitk > 1 as above, with
+ * work of splitk*(M+1)*N floats. */
+int cgfds_gemm_bf16_colsum(int M, int N, int K, const void *A, long lda, const void *G, long ldg,
+                           float *C32, long ldc32, float *csum, int splitk, float *work,
+                           void *stream);
+
+/* C32 = A B + bias (A [M][K], B [K][N]) and its moment-tensor contraction: a
+ * row of C32 is N/(nk*nc) times of nk basis terms of nc channels,
+ * y[r][t][c] = sum_k m[r/rps][k] C32[r][t][k][c], rps rows to a sample.
+ * N <= 128 and a multiple of nk*nc, nk <= 8. */
+int cgfds_gemm_bf16_mt(int M, int N, int K, const void *A, long lda, const void *B, long ldb,
+                       const float *bias, float *C32, long ldc32, int nk, int nc, int rps,
+                       const float *m, float *y, void *stream);
+
 /* out[n] = sum over m of G[m][n] (bf16 G, FP32 sums), rows cut into `splits`
  * ranges whose partials (work: splits*N floats) are summed in a fixed order. */
 int cgfds_colsum_bf16(int M, int N, const void *G, long ldg, float *out, int splits, float *work,
@@ -55,6 +70,12 @@ int cgfds_loss_grad(int nsamp, long n, const float *Y, const float *T, const flo
 int cgfds_adam(long n, float *w, float *m, float *v, const float *g, void *w16, float lr,
                float b1, float b2, float c1, float c2, float bc1, float bc2, float eps,
                void *stream);
+
+/* The same step on `count` tensors in one launch for each 32 of them: n, w, m,
+ * v, g and w16 are arrays of count entries on the host (w16's may be null). */
+int cgfds_adam_multi(int count, const long *n, float *const *w, float *const *m, float *const *v,
+                     const float *const *g, void *const *w16, float lr, float b1, float b2,
+                     float c1, float c2, float bc1, float bc2, float eps, void *stream);
 
 /* Moment-tensor contraction of basis waveforms (the seismograms are linear
  * in the moment tensor): y[b][t][c] = sum_k m[b][k] g[b][t][k][c] for

@@ -1,0 +1,107 @@
+"""GPU: the surrogate's products where their tiles, block orders and stores end:
+each tile size with rows, columns and contractions short of it, the row and the
+split order, masks and bf16 outputs on and off 16-byte rows, the column sums and
+the moment-tensor contraction formed beside a product, and Adam on a list.
+
+Sums of K bf16 products in FP32 differ from the exact ones by at most
+K 2^-23 times the sum of their magnitudes (each addition rounds once, in any
+order); a bf16 result by another 2^-8 of itself."""
+import numpy as np
+import pytest
+
+pytestmark = pytest.mark.gpu
+
+torch = pytest.importorskip("torch")
+
+
+def _bf(rng, r, c, ld=None):
+    t = torch.zeros((r, ld or c), dtype=torch.bfloat16, device="cuda:0")
+    t[:, :c] = torch.from_numpy(rng.standard_normal((r, c)).astype(np.float32)).to("cuda:0")
+    return t
+
+
+def _exact(a, b):
+    a, b = a.double().cpu(), b.double().cpu()
+    return a @ b, a.abs() @ b.abs()
+
+
+# rows, columns, contraction: 64 x 32, 64 x 64 and 128 x 128 tiles, the last with
+# 8 row tiles an XCD and more, and remainders of each
+SHAPES = [(8, 8, 8), (72, 40, 136), (520, 2056, 72), (1032, 4104, 40), (8200, 264, 200),
+          (131080, 136, 72)]
+
+
+@pytest.mark.parametrize("transB", [0, 1])
+@pytest.mark.parametrize("M,N,K", SHAPES)
+def test_bf16_output_and_mask(M, N, K, transB):
+    from cgfd3d_amd import surrogate as sg
+    rng = np.random.default_rng(M + N + K)
+    a = _bf(rng, M, K)
+    b = _bf(rng, N, K) if transB else _bf(rng, K, N)
+    bias = torch.from_numpy(rng.standard_normal(N).astype(np.float32)).to("cuda:0")
+    want, mag = _exact(a, b.t() if transB else b)
+    lim = K * 2.0 ** -23 * mag
+    for ld in (N, N + 8, N + 4):                 # the last: rows off 16 bytes
+        mask = _bf(rng, M, N, ld)
+        out = torch.full((M, ld), 7.0, dtype=torch.bfloat16, device="cuda:0")
+        sg.gemm(M, N, K, a, K, 0, b, b.shape[1], transB, epi=sg.EPI_MASK, mask=mask, ldm=ld,
+                C16=out, ldc16=ld)
+        w = torch.where(mask[:, :N].cpu() > 0, want, torch.zeros(()).double())
+        assert ((out[:, :N].double().cpu() - w).abs() <= lim + 2.0 ** -8 * w.abs()).all()
+        assert bool((out[:, N:] == 7.0).all())
+        sg.gemm(M, N, K, a, K, 0, b, b.shape[1], transB, bias=bias, epi=sg.EPI_RELU, C16=out,
+                ldc16=ld)
+        w = (want + bias.double().cpu()).clamp(min=0)
+        l2 = lim + 2.0 ** -23 * (mag + bias.double().cpu().abs())
+        assert ((out[:, :N].double().cpu() - w).abs() <= l2 + 2.0 ** -8 * w.abs()).all()
+        assert bool((out[:, N:] == 7.0).all())
+
+
+@pytest.mark.parametrize("splitk", [1, 5, 8, 19, 128])
+@pytest.mark.parametrize("M,N,K", [(8, 8, 64), (136, 72, 4104), (32, 520, 1000), (256, 2056, 264)])
+def test_products_with_column_sums(M, N, K, splitk):
+    from cgfd3d_amd import surrogate as sg
+    rng = np.random.default_rng(M + N + K)
+    a, g = _bf(rng, K, M), _bf(rng, K, N)
+    c = torch.empty((M, N), device="cuda:0")
+    s = torch.empty(N, device="cuda:0")
+    work = torch.empty(splitk * (M + 1) * N, device="cuda:0")
+    sg.gemm_colsum(M, N, K, a, M, g, N, c, s, splitk, work)
+    want, mag = _exact(a.t(), g)
+    assert ((c.double().cpu() - want).abs() <= K * 2.0 ** -23 * mag).all()
+    g = g.double().cpu()
+    assert ((s.double().cpu() - g.sum(0)).abs() <= K * 2.0 ** -23 * g.abs().sum(0)).all()
+
+
+@pytest.mark.parametrize("nk,nc,times", [(6, 3, 4), (1, 8, 1), (8, 1, 16), (2, 4, 1)])
+@pytest.mark.parametrize("nsamp,rps", [(8, 8), (40, 40), (72, 1024)])
+def test_contraction_beside_the_product(nsamp, rps, nk, nc, times):
+    """Both outputs are those of the product and the contraction apart, bit for bit."""
+    from cgfd3d_amd import surrogate as sg
+    M, N, K = nsamp * rps, nk * nc * times, 136
+    rng = np.random.default_rng(M + N)
+    a, b = _bf(rng, M, K), _bf(rng, K, N)
+    f = lambda *n: torch.from_numpy(rng.standard_normal(n).astype(np.float32)).to("cuda:0")
+    bias, m = f(N), f(nsamp, nk)
+    c, c2 = torch.empty((M, N), device="cuda:0"), torch.empty((M, N), device="cuda:0")
+    y, y2 = torch.empty(M * N // nk, device="cuda:0"), torch.empty(M * N // nk, device="cuda:0")
+    sg.gemm_mt(M, N, K, a, b, bias, c, nk, nc, rps, m, y)
+    sg.gemm(M, N, K, a, K, 0, b, N, 0, bias=bias, C32=c2, ldc32=N)
+    sg.mt_contract(nsamp, rps * times, nc, nk, m, c2, y2)
+    assert torch.equal(c, c2) and torch.equal(y, y2)
+
+
+@pytest.mark.parametrize("sizes", [(1,), (1023, 1024, 1025, 7), tuple(range(1, 40))])
+def test_adam_on_a_list(sizes):
+    from cgfd3d_amd import surrogate as sg
+    rng = np.random.default_rng(len(sizes))
+    f = lambda n: torch.from_numpy(rng.random(n, dtype=np.float32)).to("cuda:0")
+    one = [[f(n), f(n), f(n), f(n),
+            torch.empty(n, dtype=torch.bfloat16, device="cuda:0") if i % 2 else None]
+           for i, n in enumerate(sizes)]
+    many = [[None if t is None else t.clone() for t in q] for q in one]
+    for q in one:
+        sg.adam(*q, 1e-3, 3)
+    sg.adam_multi(many, 1e-3, 3)
+    for p, q in zip(one, many):
+        assert all(torch.equal(s, t) for s, t in zip(p, q) if s is not None)
