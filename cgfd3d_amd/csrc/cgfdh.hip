@@ -1212,60 +1212,106 @@ static void launch_stage(cgfdh_solver* s, hipStream_t stream, const StageParams&
 // then the pre/end swap.  ev (optional) gets a record before the first stage
 // and one after the last; it_off (optional) is a device step offset added to
 // it, for graph replays of a captured cycle.
-// ablexp sponge, bdry_ablexp_apply (bdry_t.c:840-890): every component of
-// w_end at the points of one block times min(Ex[i], Ey[j], Ez[k]); the blocks
-// are launched one after another in the reference's order, so a point that
-// two blocks share is damped twice, as there
-__global__ void ablexp_kernel(float* __restrict__ w, long vol, int nw, int nx, long ss,
-                              const float* __restrict__ Ex, const float* __restrict__ Ey,
-                              const float* __restrict__ Ez, int i1, int ni, int j1, int nj,
-                              int k1, long npt)
-{
-  const long t = (long)blockIdx.x * blockDim.x + threadIdx.x;
-  if (t >= npt) return;
-  const long r = t / ni;
-  const int i = i1 + (int)(t - r * ni);
-  const int k = k1 + (int)(r / nj);
-  const int j = j1 + (int)(r - (long)(k - k1) * nj);
-  float mask = Ex[i] < Ey[j] ? Ex[i] : Ey[j];
-  if (mask > Ez[k]) mask = Ez[k];
-  const long p = (long)i + (long)j * nx + (long)k * ss;
-  for (int c = 0; c < nw; c++) w[c * vol + p] *= mask;
-}
+// Graves-Qs attenuation and the ablexp sponge in one pass over w_end, every
+// component of the points that either touches read and written once (two
+// kernels and a launch for each sponge block before: 217x205x133 169 us a
+// step, 114 in one).
+//
+// Graves-Qs, sv_curv_col_el_graves_Qs (sv_curv_col_el.c:638-667): physical points
+// times exp(coef / Qs), coef = -pi f dt.  The exponential is evaluated in double
+// and rounded to float (correctly rounded but for rare double-rounding cases);
+// the reference's libm expf differs from it by one ulp on a few inputs in 10^5.
+//
+// Sponge, bdry_ablexp_apply (bdry_t.c:840-890): the points of each block times
+// min(Ex[i], Ey[j], Ez[k]), in the reference's order of the blocks, so a point
+// that two of them share is damped twice, as there.
+struct DampParams {
+  float* w;
+  long vol, ss;
+  int nw, nx;
+  const float* qs;                 // null without Graves-Qs
+  float coef;
+  int ni, nj, nk;                  // physical points
+  const float *Ex, *Ey, *Ez;
+  int nblk, blk[6][6];             // i1, i2, j1, j2, k1, k2
+  int i0, i1, j0, j1, k0, k1;      // the box of all points concerned
+};
 
-// Graves-Qs attenuation, sv_curv_col_el_graves_Qs (sv_curv_col_el.c:638-667):
-// every component at physical points times exp(coef / Qs), coef = -pi f dt.
-// The exponential is evaluated in double and rounded to float (correctly
-// rounded but for rare double-rounding cases); the reference's libm expf
-// differs from it by one ulp on a few inputs in 10^5.
-__global__ void graves_qs_kernel(float* __restrict__ w, long vol, int nw, int nx, long ss,
-                                 const float* __restrict__ qs, float coef, int ni, int nj,
-                                 long npt)
+__device__ __forceinline__ void damp_point(const DampParams& D, int i, int j, int k)
 {
-  const long t = (long)blockIdx.x * blockDim.x + threadIdx.x;
-  if (t >= npt) return;
-  const long r = t / ni;
-  const int i = 3 + (int)(t - r * ni);
-  const int k = 3 + (int)(r / nj);
-  const int j = 3 + (int)(r - (long)(k - 3) * nj);
-  const long p = (long)i + (long)j * nx + (long)k * ss;
-  const float att = (float)exp((double)(coef / qs[p]));
-  for (int c = 0; c < nw; c++) w[c * vol + p] *= att;
-}
-
-static void enqueue_ablexp(cgfdh_solver* s, hipStream_t st)
-{
-  const float* Ex = s->abl;
-  const float* Ey = s->abl + s->nx;
-  const float* Ez = s->abl + s->nx + s->ny;
-  for (int n = 0; n < s->abl_n; n++) {
-    const int* b = s->abl_blk[n];
-    const int ni = b[1] - b[0] + 1, nj = b[3] - b[2] + 1, nk = b[5] - b[4] + 1;
-    const long npt = (long)ni * nj * nk;
-    hipLaunchKernelGGL(ablexp_kernel, dim3((unsigned)((npt + 255) / 256)), dim3(256), 0, st,
-                       s->lvl[3], s->vol, s->nw, s->px, s->ss, Ex, Ey, Ez, b[0], ni, b[2], nj,
-                       b[4], npt);
+  const long p = (long)i + (long)j * D.nx + (long)k * D.ss;
+  int n = 0;
+  const bool q = D.qs && i >= 3 && i < 3 + D.ni && j >= 3 && j < 3 + D.nj && k >= 3 &&
+                 k < 3 + D.nk;
+#pragma unroll
+  for (int b = 0; b < 6; b++) {
+    const int* r = D.blk[b];
+    if (b < D.nblk && i >= r[0] && i <= r[1] && j >= r[2] && j <= r[3] && k >= r[4] && k <= r[5])
+      n++;
   }
+  if (!q && !n) return;
+  float att = 1.0f, mask = 1.0f;
+  if (q) att = (float)exp((double)(D.coef / D.qs[p]));
+  if (n) {
+    mask = D.Ex[i] < D.Ey[j] ? D.Ex[i] : D.Ey[j];
+    if (mask > D.Ez[k]) mask = D.Ez[k];
+  }
+  for (int c0 = 0; c0 < D.nw; c0 += 9) {
+    float v[9];
+#pragma unroll
+    for (int c = 0; c < 9; c++)
+      if (c0 + c < D.nw) v[c] = D.w[(c0 + c) * D.vol + p];
+#pragma unroll
+    for (int c = 0; c < 9; c++) {
+      if (q) v[c] *= att;
+      for (int b = 0; b < n; b++) v[c] *= mask;
+    }
+#pragma unroll
+    for (int c = 0; c < 9; c++)
+      if (c0 + c < D.nw) D.w[(c0 + c) * D.vol + p] = v[c];
+  }
+}
+
+__global__ void __launch_bounds__(256) damp_kernel(DampParams D)
+{
+  const int i = D.i0 + blockIdx.x * 64 + threadIdx.x;
+  if (i > D.i1) return;
+  for (int k = D.k0 + blockIdx.z; k <= D.k1; k += gridDim.z)
+    for (int j = D.j0 + blockIdx.y * 4 + threadIdx.y; j <= D.j1; j += gridDim.y * 4)
+      damp_point(D, i, j, k);
+}
+
+static void enqueue_damp(cgfdh_solver* s, hipStream_t st)
+{
+  DampParams D;
+  memset(&D, 0, sizeof D);
+  D.w = s->lvl[3];
+  D.vol = s->vol; D.ss = s->ss; D.nw = s->nw; D.nx = s->px;
+  D.qs = s->qs; D.coef = s->qs_coef;
+  D.ni = s->d.ni; D.nj = s->d.nj; D.nk = s->d.nk;
+  D.Ex = s->abl;
+  D.Ey = s->abl ? s->abl + s->nx : nullptr;
+  D.Ez = s->abl ? s->abl + s->nx + s->ny : nullptr;
+  D.nblk = s->abl_n;
+  memcpy(D.blk, s->abl_blk, sizeof D.blk);
+  int lo[3] = {s->nx, s->ny, s->nz}, hi[3] = {-1, -1, -1};
+  if (s->qs) {
+    const int n[3] = {s->d.ni, s->d.nj, s->d.nk};
+    for (int a = 0; a < 3; a++) {
+      lo[a] = 3;
+      hi[a] = 2 + n[a];
+    }
+  }
+  for (int b = 0; b < s->abl_n; b++)
+    for (int a = 0; a < 3; a++) {
+      lo[a] = std::min(lo[a], s->abl_blk[b][2 * a]);
+      hi[a] = std::max(hi[a], s->abl_blk[b][2 * a + 1]);
+    }
+  D.i0 = lo[0]; D.i1 = hi[0]; D.j0 = lo[1]; D.j1 = hi[1]; D.k0 = lo[2]; D.k1 = hi[2];
+  hipLaunchKernelGGL(damp_kernel,
+                     dim3((hi[0] - lo[0] + 64) / 64, std::min((hi[1] - lo[1] + 4) / 4, 65535),
+                          std::min(hi[2] - lo[2] + 1, 65535)),
+                     dim3(64, 4), 0, st, D);
 }
 
 // what follows the four stages of step it (drv_rk_curv_col.c:414-544): the
@@ -1277,13 +1323,8 @@ static int enqueue_post_step(cgfdh_solver* s, hipStream_t st, int it, const int*
     hipLaunchKernelGGL(vis_free_kernel, dim3((s->d.ni + 255) / 256, s->d.nj), dim3(256), 0, st,
                        s->lvl[3], s->mats + 27 * s->ss, s->d.ni, s->d.nj, s->px, s->ss, s->vol,
                        s->nk2);
-  if (s->qs) {   // after the last stage's combine, drv_rk_curv_col.c:414-416
-    const long npt = (long)s->d.ni * s->d.nj * s->d.nk;
-    hipLaunchKernelGGL(graves_qs_kernel, dim3((unsigned)((npt + 255) / 256)), dim3(256), 0, st,
-                       s->lvl[3], s->vol, s->nw, s->px, s->ss, s->qs, s->qs_coef, s->d.ni,
-                       s->d.nj, npt);
-  }
-  if (s->abl_n) enqueue_ablexp(s, st);   // drv_rk_curv_col.c:482-486
+  // drv_rk_curv_col.c:414-416 and 482-486
+  if (s->qs || s->abl_n) enqueue_damp(s, st);
   if (s->pg)   // drv_rk_curv_col.c:492-495, before the pre/end swap
     hipLaunchKernelGGL(pg_kernel, dim3((s->d.ni + 255) / 256, s->d.nj), dim3(256), 0, st,
                        s->lvl[3], s->lvl[0], s->pg, s->pg + 15 * s->ss, s->d.ni, s->d.nj, s->px,
