@@ -57,8 +57,8 @@ KERNELS = [
     ("stage_interior_ldsp8", "stage_interior_ldsp_kernel<TY=8> + shell kernels"),
     ("stage_interior_phased_w3", "stage_interior_phased_kernel<BY=4, 3 waves/SIMD> + "
                                  "shell kernels"),
-    ("stage_rows_phased", "stage_rows_phased_kernel<BY=4> (whole rows, PML folded in) + "
-                          "free-surface rows"),
+    ("stage_rows_phased", "stage_tile_kernel<TY=8> (plane tiles of whole rows through LDS, PML "
+                          "folded in) + free-surface rows"),
     ("stage_interior_phased_shellp", "stage_interior_phased_kernel<BY=4> + "
                                      "stage_shellp_kernel (phased PML slabs) + free-surface rows"),
     ("stage_rows_lds", "stage_rows_lds_kernel<BY=4> (whole rows, PML folded in, non-stencil "
@@ -436,8 +436,7 @@ def main():
     ap.add_argument("--steps", type=int, default=20)
     ap.add_argument("--warmup", type=int, default=3)
     ap.add_argument("--variant", type=int, default=None,
-                    help="stage kernels (default: the engine's choice for the medium, 16 "
-                         "isotropic, VTI and visco-elastic, 18 anisotropic): 0 per-point, 1 "
+                    help="stage kernels (default: 16): 0 per-point, 1 "
                          "tiled, 2/3 z-marching interior + "
                          "shell, 4/5 per-point interior (64x4 / 64x2) + shell, 6/7 "
                          "x-vectorised interior (2 / 4 points per thread) + shell, 8/9 "
@@ -445,10 +444,10 @@ def main():
                          "per-point interior marching 2 / 4 planes per block + shell, 12 "
                          "two-phase per-point interior + shell, 13 the same with the RK "
                          "combine loads last, 14 LDS-tiled interior with phased loads + shell, "
-                         "15 variant 12 built for 3 waves per SIMD, 16 whole-row two-phase "
-                         "kernel with the PML faces folded in, 17 variant 12 with a two-phase "
-                         "shell, 18 variant 16 with the operands that have no stencil loaded "
-                         "straight to LDS (4 waves per SIMD); with --workload batch a "
+                         "15 variant 12 built for 3 waves per SIMD, 16 plane "
+                         "tiles of whole rows through LDS with the PML faces folded in, 17 "
+                         "variant 12 with a two-phase shell, 18 whole-row two-phase kernel with "
+                         "the operands that have no stencil loaded straight to LDS; with --workload batch a "
                          "given variant serves every grid and the autotune is skipped")
     ap.add_argument("--workload", default="iso",
                     choices=["iso", "vti", "aniso", "visco", "batch", "media"])

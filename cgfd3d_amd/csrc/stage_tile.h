@@ -15,9 +15,9 @@
 //  * rows start on 128-byte lines, so a wave's load is two lines, not three;
 //  * registers are kept to 128, 4 waves a SIMD in two blocks a compute unit,
 //    whose loads cover each other's arithmetic.
-// 95 vector memory instructions a point are left and the traffic is within 5 %
-// of the least (plane by plane), 4.2 TB/s on it.  600x600x300 isotropic, ms a
-// step, before and now: 29.7, 23.3; without PML 24.7, 19.4; 400x400x200 VTI
+// 95 vector memory instructions a point are left and 1.14 times the algorithmic
+// traffic (the two-phase kernel: 1.15), 4.7 TB/s on it.  600x600x300 isotropic, ms
+// a step, before and now: 29.7, 23.3; without PML 24.7, 19.4; 400x400x200 VTI
 // 10.1, 8.3; anisotropic 11.8, 9.9; visco-elastic (3 bodies) 22.7, 15.9.
 #pragma once
 #include <type_traits>

@@ -534,15 +534,16 @@ int cgfdh_last_timing(cgfdh_solver *s, double *run_ms, double *stage_ms,
  * (all loads, then the arithmetic; 13 loads the RK combine inputs last),
  * 14 = LDS-tiled plane kernel with the same phased loads, 15 = variant 12
  * compiled for 3 waves per SIMD; 2..15 run the per-point kernel on the PML
- * and free-surface shell; 16 = the two-phase kernel over whole rows with the
- * PML faces folded in (free-surface rows on the per-point kernel); 17 = the
+ * and free-surface shell; 16 = plane tiles of 64x8 points over whole rows,
+ * operands through LDS, with the PML faces folded in (free-surface rows on the
+ * per-point kernel; volumes above 536 M points, cgfdh_onestage and the fused
+ * batch cycle on the two-phase kernel over whole rows); 17 = the
  * two-phase interior kernel on the tiles clear of every PML face plus a
  * shell kernel that requests each PML slab's memory variables first; 18 =
- * variant 16 with the metric, medium, slowness and RK combine inputs loaded
- * straight to LDS (global_load_lds), so the stencil values alone hold
- * registers and four waves fit per SIMD.
- * Default 16 for the isotropic, VTI and visco-elastic media, 18 for the
- * anisotropic medium (whose 21 coefficients otherwise hold registers).
+ * the two-phase kernel over whole rows with the metric, medium, slowness and
+ * RK combine inputs loaded straight to LDS (global_load_lds), so the stencil
+ * values alone hold registers and four waves fit per SIMD.
+ * Default 16 for every medium.
  * Variants 1..3 exist for the isotropic medium only; the visco-elastic
  * medium has 0, 4, 5, 8..11 and 16.
  * All variants produce identical bits. */
