@@ -496,14 +496,18 @@ static int copy_rows(cgfdh_solver* s, float* dev, int per, float* host, long nro
     HIPCHK(hipStreamSynchronize(s->stream));
     return CGFDH_OK;
   }
-  const long rows = std::max(1l, std::min(nrow, (1l << 24) / len));
+  const long cap = 1l << 24;
+  const long rows = std::max(1l, std::min(nrow, cap / len));
   if (s->stage_n < (size_t)(rows * len)) {
     HIPCHK(hipStreamSynchronize(s->stream));
     if (s->stage) HIPCHK(hipFree(s->stage));
     s->stage = nullptr;
     s->stage_n = 0;
-    HIPCHK(hipMalloc((void**)&s->stage, rows * len * sizeof(float)));
-    s->stage_n = rows * len;
+    // room for the ten volumes of the metric at once, so that a small solver's
+    // setters do not grow it one after another
+    const long n = std::max(rows * len, std::min(cap, 10l * s->nx * s->ny * s->nz));
+    HIPCHK(hipMalloc((void**)&s->stage, n * sizeof(float)));
+    s->stage_n = n;
   }
   for (long r = 0; r < nrow; r += rows) {
     const long n = std::min(rows, nrow - r);
@@ -1207,11 +1211,6 @@ static void launch_stage(cgfdh_solver* s, hipStream_t stream, const StageParams&
   }
 }
 
-// one RK4 step of solver s on stream st (drv_rk_curv_col.c:167-544): four fused
-// stages, the visco-elastic surface rotation, peak ground motion, receivers,
-// then the pre/end swap.  ev (optional) gets a record before the first stage
-// and one after the last; it_off (optional) is a device step offset added to
-// it, for graph replays of a captured cycle.
 // Graves-Qs attenuation and the ablexp sponge in one pass over w_end, every
 // component of the points that either touches read and written once (two
 // kernels and a launch for each sponge block before: 217x205x133 169 us a
@@ -1341,6 +1340,11 @@ static int enqueue_post_step(cgfdh_solver* s, hipStream_t st, int it, const int*
   return CGFDH_OK;
 }
 
+// one RK4 step of solver s on stream st (drv_rk_curv_col.c:167-544): four fused
+// stages, the visco-elastic surface rotation, peak ground motion, receivers,
+// then the pre/end swap.  ev (optional) gets a record before the first stage
+// and one after the last; it_off (optional) is a device step offset added to
+// it, for graph replays of a captured cycle.
 static int enqueue_step(cgfdh_solver* s, hipStream_t st, int it, const int* it_off,
                         hipEvent_t* ev)
 {
