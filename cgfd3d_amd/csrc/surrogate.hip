@@ -110,16 +110,25 @@ typedef uint16_t u16x8 __attribute__((ext_vector_type(8)));
 
 constexpr unsigned OUT = ~15u;   // an offset past every operand: loads zeros
 
+__device__ const uint16_t zero16[8] __attribute__((aligned(16))) = {};
+
 // One operand's tile, loaded straight to LDS 16 bytes a lane.  KC: the
 // contraction index is the contiguous one, R rows of BK; otherwise BK rows of R.
 // Inside a row the 16-byte chunks are exchanged by an exclusive or with bits of
 // the row, so that the 16 rows (KC) or the 4 x 2 rows (not KC) a fragment reads
-// at one chunk lie in different banks.
-template <bool KC, int R, int BK, int NT> struct Operand {
+// at one chunk lie in different banks.  WIDE: leading dimensions beyond the
+// 32-bit offsets, by 64-bit addresses.
+template <bool KC, int R, int BK, int NT, bool WIDE> struct Operand {
   static constexpr int ROWS = KC ? R : BK, COLS = KC ? BK : R;
   static constexpr int CH = COLS / 8;             // chunks of a row
   static constexpr int N = ROWS * CH / NT;        // loads of a thread
   static_assert(ROWS * CH % NT == 0 && (CH & (CH - 1)) == 0, "");
+
+  // whether the rows of a wave's load are too far apart for a lane's 32-bit
+  // byte offset: 64 / CH rows, 16 of a tile of 32 columns, so from leading
+  // dimensions of 143 million on there and 307 or 716 million elsewhere
+  static bool too_wide(long ld) { return ld > (long)(OUT / 2 - 8 * CH) / (64 / CH - 1); }
+
   static __device__ __forceinline__ int swz(int r)
   {
     if (KC) return r & (CH < 8 ? CH - 1 : 7);
@@ -139,9 +148,16 @@ template <bool KC, int R, int BK, int NT> struct Operand {
       // most 16 rows) in the 32-bit offset
       const int rw = (i * NT + w * 64) / CH;
       const int id = i * NT + t, r = id / CH, c = (id % CH) ^ swz(r);
+      const bool ok = KC ? (r0 + r < nr && k + 8 * c < ke) : (k + r < ke && r0 + 8 * c < nr);
+      if (WIDE) {
+        const uint16_t* q = ok ? p + (r * ld + 8 * c) : zero16;
+        __builtin_amdgcn_global_load_lds(
+            (const __attribute__((address_space(1))) void*)q,
+            (__attribute__((address_space(3))) void*)(lds + (long)(i * NT + w * 64) * 8), 16, 0, 0);
+        continue;
+      }
       const __amdgpu_buffer_rsrc_t q = __builtin_amdgcn_make_buffer_rsrc(
           (void*)(p + rw * ld), 0, (int)0xfffffff0, 0x00020000);
-      const bool ok = KC ? (r0 + r < nr && k + 8 * c < ke) : (k + r < ke && r0 + 8 * c < nr);
       const unsigned off = ok ? (unsigned)((r - rw) * (unsigned)ld + 8 * c) * 2u : OUT;
       __builtin_amdgcn_raw_ptr_buffer_load_lds(
           q, (__attribute__((address_space(3))) void*)(lds + (long)(i * NT + w * 64) * 8), 16,
@@ -179,12 +195,12 @@ template <bool KC, int R, int BK, int NT> struct Operand {
 // NS stages of BK in a ring, NS - 1 of them in flight.  The products are formed
 // as (B^T A^T): a lane then holds 4 neighbouring columns of one row of C, which
 // leave in one 16- or 8-byte store.
-template <int TA, int TB, int BM, int BN, int BK, int NS, int WM, int WN>
+template <int TA, int TB, int BM, int BN, int BK, int NS, int WM, int WN, bool WIDE = false>
 __global__ __launch_bounds__(64 * WM * WN) void gemm_bf16_kernel(GemmArgs g)
 {
   constexpr int NT = 64 * WM * WN;
-  using OA = Operand<!TA, BM, BK, NT>;
-  using OB = Operand<TB, BN, BK, NT>;
+  using OA = Operand<!TA, BM, BK, NT, WIDE>;
+  using OB = Operand<TB, BN, BK, NT, WIDE>;
   constexpr int FM = BM / WM / 16, FN = BN / WN / 16;
   // the ring; behind the products the waves' output rows
   constexpr int RING = NS * (BM + BN) * BK, ROWS = BM * BN + 8 * BM * WN;
@@ -663,9 +679,20 @@ static int gemm_launch(const char* name, GemmArgs g, int transA, int transB, int
     return (long)g.mt * g.nt * (g.order == ORD_SPLIT ? (S + 7) / 8 * 8 : S);
   };
   long blocks = 0;
+  // whether an operand's rows are too far apart for a tile's 32-bit offsets
+  auto too_wide = [&](auto bm, auto bn, auto bk) {
+    constexpr int BM = decltype(bm)::value, BN = decltype(bn)::value, BK = decltype(bk)::value;
+    return (transA ? Operand<false, BM, BK, 256, false>::too_wide(g.lda)
+                   : Operand<true, BM, BK, 256, false>::too_wide(g.lda)) ||
+           (transB ? Operand<true, BN, BK, 256, false>::too_wide(g.ldb)
+                   : Operand<false, BN, BK, 256, false>::too_wide(g.ldb));
+  };
+  bool wide = false;
   auto launch = [&](auto bm, auto bn, auto bk, auto ns, auto wm) {
     constexpr int BM = decltype(bm)::value, BN = decltype(bn)::value, BK = decltype(bk)::value,
                   NS = decltype(ns)::value, WM = decltype(wm)::value;
+    wide = too_wide(bm, bn, bk);
+    if (wide) return;
     blocks = shape(BM, BN);
     if (blocks > 0x7fffffffl) return;
     const dim3 grid((unsigned)blocks), blk(128 * WM);
@@ -692,13 +719,31 @@ static int gemm_launch(const char* name, GemmArgs g, int transA, int transB, int
     launch(CGFDS_I(128), CGFDS_I(128), CGFDS_I(64), CGFDS_I(2), CGFDS_I(4));
   } else if (g.y) {
     // the contraction needs whole rows in a block
-    blocks = shape(64, 128);
-    hipLaunchKernelGGL((gemm_bf16_kernel<0, 0, 64, 128, 64, 3, 2, 2>), dim3((unsigned)blocks),
-                       dim3(256), 0, st, g);
+    wide = too_wide(CGFDS_I(64), CGFDS_I(128), CGFDS_I(64));
+    if (!wide) {
+      blocks = shape(64, 128);
+      hipLaunchKernelGGL((gemm_bf16_kernel<0, 0, 64, 128, 64, 3, 2, 2>), dim3((unsigned)blocks),
+                         dim3(256), 0, st, g);
+    }
   } else if (mid >= 256) {
     launch(CGFDS_I(64), CGFDS_I(64), CGFDS_I(64), CGFDS_I(3), CGFDS_I(2));
   } else {
     launch(CGFDS_I(64), CGFDS_I(32), CGFDS_I(128), CGFDS_I(4), CGFDS_I(2));
+  }
+  if (wide) {
+    // one tile serves them: matrices of gigabytes of which few values are read
+    blocks = g.y ? shape(64, 128) : shape(64, 32);
+    const dim3 grid((unsigned)blocks), blk(256);
+#define CGFDS_W(TA, TB) \
+  hipLaunchKernelGGL((gemm_bf16_kernel<TA, TB, 64, 32, 128, 4, 2, 2, true>), grid, blk, 0, st, g)
+    if (blocks > 0x7fffffffl) return bad("more than 2^31 - 1 tiles");
+    if (g.y)
+      hipLaunchKernelGGL((gemm_bf16_kernel<0, 0, 64, 128, 64, 3, 2, 2, true>), grid, blk, 0, st, g);
+    else if (form == 0) CGFDS_W(0, 0);
+    else if (form == 1) CGFDS_W(0, 1);
+    else if (form == 2) CGFDS_W(1, 0);
+    else CGFDS_W(1, 1);
+#undef CGFDS_W
   }
 #undef CGFDS_I
   if (blocks > 0x7fffffffl) return bad("more than 2^31 - 1 tiles");

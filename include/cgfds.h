@@ -28,7 +28,8 @@ extern "C" {
  * accumulation.  opA = A stored [M][lda] or, transA, A^T of A stored
  * [K][lda]; opB = B stored [K][ldb] or, transB, B^T of B stored [N][ldb].
  * The epilogue's v goes to C32 (FP32, optional) and/or C16 (bf16, optional).
- * M, N, K, lda, ldb must be multiples of 8 and A, B 16-byte aligned.
+ * M, N, K, lda, ldb must be multiples of 8 and A, B 16-byte aligned; lda and
+ * ldb have no upper limit.
  * splitk > 1 splits the K range over that many workgroup layers whose FP32
  * partials (work: splitk*M*N floats) are summed in a fixed order into C32;
  * it requires EPI_NONE, no bias and no C16. */

@@ -91,6 +91,56 @@ def test_contraction_beside_the_product(nsamp, rps, nk, nc, times):
     assert torch.equal(c, c2) and torch.equal(y, y2)
 
 
+def _spread(rng, r, c, ld):
+    """r rows of c values ld apart; what lies between them is not touched."""
+    t = torch.empty(r * ld, dtype=torch.bfloat16, device="cuda:0").view(r, ld)
+    t[:, :c] = torch.from_numpy(rng.standard_normal((r, c)).astype(np.float32)).to("cuda:0")
+    return t
+
+
+# leading dimensions just past the 32-bit byte offsets of 16, 8 and 4 rows
+W16, W8, W4 = 143165584, 306783384, 715827888
+
+
+@pytest.mark.parametrize("M,N,K,transA,transB,lda,ldb", [
+    (8, 8, 16, 0, 0, 16, W16), (8, 8, 16, 0, 0, W4, 8), (8, 8, 16, 0, 1, 16, W4),
+    (8, 8, 16, 1, 0, W8, 8), (32768, 8, 8, 1, 0, W4, 8)])
+def test_rows_past_32_bit_offsets(M, N, K, transA, transB, lda, ldb):
+    from cgfd3d_amd import surrogate as sg
+    rng = np.random.default_rng(M + lda % 97)
+    a = _spread(rng, K, M, lda) if transA else _spread(rng, M, K, lda)
+    b = _spread(rng, N, K, ldb) if transB else _spread(rng, K, N, ldb)
+    c = torch.empty((M, N), device="cuda:0")
+    sg.gemm(M, N, K, a, lda, transA, b, ldb, transB, C32=c, ldc32=N)
+    want, mag = _exact(a[:, :M].t() if transA else a[:, :K], b[:, :K].t() if transB else b[:, :N])
+    assert ((c.double().cpu() - want).abs() <= K * 2.0 ** -23 * mag).all()
+    if transA:
+        s, work = torch.empty(N, device="cuda:0"), torch.empty((M + 1) * N, device="cuda:0")
+        sg.gemm_colsum(M, N, K, a, lda, b, ldb, c, s, 1, work)
+        assert ((c.double().cpu() - want).abs() <= K * 2.0 ** -23 * mag).all()
+        g = b[:, :N].double().cpu()
+        assert ((s.double().cpu() - g.sum(0)).abs() <= K * 2.0 ** -23 * g.abs().sum(0)).all()
+
+
+def test_contraction_of_rows_past_32_bit_offsets():
+    from cgfd3d_amd import surrogate as sg
+    from cgfd3d_amd._lib import check, lib
+    M, N, K, nk, nc, ldb = 8, 72, 8, 6, 3, W4
+    rng = np.random.default_rng(5)
+    a, b = _bf(rng, M, K), _spread(rng, K, N, ldb)
+    m = torch.from_numpy(rng.standard_normal((1, nk)).astype(np.float32)).to("cuda:0")
+    bias = torch.zeros(N, device="cuda:0")
+    c, y = torch.empty((M, N), device="cuda:0"), torch.empty(M * N // nk, device="cuda:0")
+    y2 = torch.empty_like(y)
+    p = lambda t: t.data_ptr()
+    check(lib().cgfds_gemm_bf16_mt(M, N, K, p(a), K, p(b), ldb, p(bias), p(c), N, nk, nc, M, p(m),
+                                   p(y), torch.cuda.current_stream().cuda_stream), "gemm_bf16_mt")
+    want, mag = _exact(a, b[:, :N])
+    assert ((c.double().cpu() - want).abs() <= K * 2.0 ** -23 * mag).all()
+    sg.mt_contract(1, M * N // (nk * nc), nc, nk, m, c, y2)
+    assert torch.equal(y, y2)
+
+
 @pytest.mark.parametrize("sizes", [(1,), (1023, 1024, 1025, 7), tuple(range(1, 40))])
 def test_adam_on_a_list(sizes):
     from cgfd3d_amd import surrogate as sg
