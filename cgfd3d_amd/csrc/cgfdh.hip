@@ -257,6 +257,7 @@ struct cgfdh_solver {
   int abl_n = 0;
   size_t outbuf_n = 0;
   int variant = 12;              // set per medium in cgfdh_create
+  bool tile = true;              // variant 16: the tile kernel, or the two-phase one
   int tgx = 0, tgy = 0;          // tile group (0: the default)
   bool metric_set = false, medium_set = false, mats_set = false;
   // configuration generation: every setter bumps it, so a batch graph
@@ -311,6 +312,15 @@ static void set_layout(cgfdh_solver* s, bool aligned)
   s->px = aligned ? (s->nx + 31) / 32 * 32 : s->nx;
   s->ss = (long)s->px * s->ny;
   s->vol = s->ss * s->nz;
+}
+
+// whether variant 16 steps on the tile kernel, which reaches two volumes and a
+// plane on by 32-bit offsets (536 M points, the rows' padding among them).
+// CGFDH_TILE=0 (a tuning knob, read at creation): the two-phase kernel instead
+static bool tile_chosen(const cgfdh_solver* s)
+{
+  const char* e = getenv("CGFDH_TILE");
+  return !(e && e[0] == '0') && 4.0 * (2.0 * s->vol + s->ss) < 4294967280.0;
 }
 
 // the place in a device volume of a point of the reference's array
@@ -403,8 +413,11 @@ extern "C" int cgfdh_create(const cgfdh_desc* d, cgfdh_solver** out)
     for (auto& f : s->face) f = FaceHost();
     bad = alloc_all(false);
   }
-  // default stage kernel of every medium
-  s->variant = 16;
+  s->tile = tile_chosen(s);
+  // default stage kernel: where the tile kernel does not step, the anisotropic
+  // medium's best is the whole-row kernel through LDS (400x400x200: 11.96 ms a
+  // step, the two-phase kernel 12.25)
+  s->variant = d->medium_type == CGFDH_MEDIUM_ELASTIC_ANISO && !s->tile ? 18 : 16;
   if (!bad && hipStreamCreate(&s->stream) != hipSuccess) bad = 1;
   if (!bad && (hipStreamCreate(&s->stream2) != hipSuccess ||
                hipEventCreateWithFlags(&s->ev_fork, hipEventDisableTiming) != hipSuccess ||
@@ -1183,10 +1196,7 @@ static void launch_stage(cgfdh_solver* s, hipStream_t stream, const StageParams&
     (void)hipStreamWaitEvent(s->stream2, s->ev_fork, 0);
     L.shell_stream = s->stream2;
   }
-  // the tile kernel reaches two volumes and a plane on by 32-bit offsets (536 M
-  // points); larger volumes stay on the two-phase kernel
-  if (s->variant == 16 && kind != KIND_RHS && !slab_only &&
-      4.0 * (2.0 * s->vol + s->ss) < 4294967280.0) {
+  if (s->variant == 16 && s->tile && kind != KIND_RHS && !slab_only) {
     if (s->d.medium_type == CGFDH_MEDIUM_ELASTIC_VTI)
       launch_tile_vti(L, P, kind, dx, dy, dz);
     else if (s->d.medium_type == CGFDH_MEDIUM_ELASTIC_ANISO)
@@ -3282,6 +3292,7 @@ extern "C" int cgfdh_batch_autotune(cgfdh_batch* b, int it0)
 {
   if (!b) return fail(CGFDH_EINVAL, "cgfdh_batch_autotune: null batch");
   batch_drop_graph(b);
+  constexpr int TWO_PHASE = -16;
   for (size_t i = 0; i < b->sv.size(); i++) {
     cgfdh_solver* s = b->sv[i];
     int rc = ready(s, "cgfdh_batch_autotune");
@@ -3320,6 +3331,10 @@ extern "C" int cgfdh_batch_autotune(cgfdh_batch* b, int it0)
     std::vector<int> variants = visco ? std::vector<int>{4, 5, 8, 9, 16}
                                       : std::vector<int>{4, 6, 7, 8, 12, 14, 16, 18};
     if (iso) variants.push_back(3);
+    // variant 16 on both of its kernels, where the tile kernel reaches
+    const bool tile = s->tile;
+    bool bt = tile;
+    if (tile) variants.push_back(TWO_PHASE);
     const int groups[][2] = {{9, 2}, {3, 4}, {9, 8}};
     float best = 1e30f;
     int bv = s->variant, bgx = s->tgx, bgy = s->tgy;
@@ -3327,7 +3342,8 @@ extern "C" int cgfdh_batch_autotune(cgfdh_batch* b, int it0)
     for (int v : variants)
       for (auto& g : groups) {
         if (e != hipSuccess) break;
-        s->variant = v;
+        s->variant = v == TWO_PHASE ? 16 : v;
+        s->tile = tile && v != TWO_PHASE;
         s->tgx = g[0];
         s->tgy = g[1];
         float ms = 0;
@@ -3342,12 +3358,15 @@ extern "C" int cgfdh_batch_autotune(cgfdh_batch* b, int it0)
           for (auto& f : s->face)
             if (f.on) std::swap(f.aux[0], f.aux[2]);
         }
-        if (e == hipSuccess && ms < best) { best = ms; bv = v; bgx = g[0]; bgy = g[1]; }
+        if (e == hipSuccess && ms < best) {
+          best = ms; bv = s->variant; bt = s->tile; bgx = g[0]; bgy = g[1];
+        }
       }
     if (e == hipSuccess) e = copy_state(false);
     if (e == hipSuccess) e = hipStreamSynchronize(s->stream);
     (void)hipFree(save);
     s->variant = bv;
+    s->tile = bt;
     s->tgx = bgx;
     s->tgy = bgy;
     if (e != hipSuccess)

@@ -543,7 +543,9 @@ int cgfdh_last_timing(cgfdh_solver *s, double *run_ms, double *stage_ms,
  * the two-phase kernel over whole rows with the metric, medium, slowness and
  * RK combine inputs loaded straight to LDS (global_load_lds), so the stencil
  * values alone hold registers and four waves fit per SIMD.
- * Default 16 for every medium.
+ * Default 16; 18 for anisotropic volumes above 536 M points.  The environment's
+ * CGFDH_TILE=0, read by cgfdh_create, has variant 16 step on the two-phase
+ * kernel at every size.
  * Variants 1..3 exist for the isotropic medium only; the visco-elastic
  * medium has 0, 4, 5, 8..11 and 16.
  * All variants produce identical bits. */

@@ -43,3 +43,23 @@ def test_tile_edges_match_oracle(ni, nj, nk, medium):
     assert np.isfinite(w_o).all() and np.abs(w_o).max() > 0
     assert np.array_equal(w_g, np.asarray(w_o).reshape(-1))
     assert np.array_equal(a_g, np.asarray(a_o).reshape(-1))
+
+
+@pytest.mark.parametrize("medium", MEDIA)
+@pytest.mark.parametrize("ni,nj,nk", SHAPES[1::2])
+def test_two_phase_steps_match_oracle(ni, nj, nk, medium, monkeypatch):
+    """Variant 16 on the kernel that steps volumes past the tile kernel's reach."""
+    monkeypatch.setenv("CGFDH_TILE", "0")
+    test_tile_edges_match_oracle(ni, nj, nk, medium)
+
+
+@pytest.mark.parametrize("medium,nk,variant", [("iso", 500, 16), ("iso", 520, 16),
+                                               ("aniso", 490, 16), ("aniso", 520, 18)])
+def test_default_past_the_tile_kernel(medium, nk, variant):
+    """1024 x 1024 rows and planes of 506, 526 and 496: 531, 552 and 520 M points,
+    either side of two volumes and a plane of 2^32 bytes (537 M)."""
+    from cgfd3d_amd import MEDIUM_ELASTIC_ANISO, MEDIUM_ELASTIC_ISO, Solver
+    s = Solver(1018, 1018, nk, 0.004, 1, medium_type=MEDIUM_ELASTIC_ANISO if medium == "aniso"
+               else MEDIUM_ELASTIC_ISO)
+    assert s.kernel_choice()[0] == variant
+    s.close()
