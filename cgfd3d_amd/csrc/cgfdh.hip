@@ -314,13 +314,58 @@ static void set_layout(cgfdh_solver* s, bool aligned)
   s->vol = s->ss * s->nz;
 }
 
-// whether variant 16 steps on the tile kernel, which reaches two volumes and a
-// plane on by 32-bit offsets (536 M points, the rows' padding among them).
-// CGFDH_TILE=0 (a tuning knob, read at creation): the two-phase kernel instead
+// of the device volumes: the wavefield's four levels, the metric, the medium
+static long vol_bytes(const cgfdh_solver* s)
+{
+  return (4l * s->nw + 10 + s->ncmp) * s->vol * (long)sizeof(float);
+}
+
+// the last-level cache
+constexpr long LLC = 256l << 20;
+
+// the tile kernel reaches two volumes and a plane on by 32-bit offsets: 536 M
+// points, the rows' padding among them
+static bool tile_reaches(const cgfdh_solver* s)
+{
+  return 4.0 * (2.0 * s->vol + s->ss) < 4294967280.0;
+}
+
+// Whether variant 16 steps on the tile kernel (stage_tile.h) or on the two-phase
+// one (stage_interior.h).  CGFDH_TILE=0 or 1, a tuning knob read at creation, has
+// it on neither or on every grid in its reach.
 static bool tile_chosen(const cgfdh_solver* s)
 {
   const char* e = getenv("CGFDH_TILE");
-  return !(e && e[0] == '0') && 4.0 * (2.0 * s->vol + s->ss) < 4294967280.0;
+  if (!tile_reaches(s) || (e && e[0] == '0')) return false;
+  if (e && e[0] == '1') return true;
+  // On rows off the cache lines its streams past the cache gain nothing:
+  // 200x200x100 isotropic 1.69 ms a step, two-phase 1.57.
+  if (!s->lead && vol_bytes(s) > LLC) return false;
+  const cgfdh_desc& d = s->d;
+  const bool visco = d.medium_type == CGFDH_MEDIUM_VISCO_ISO;
+  // One tile a row that meets both x faces does a tile's face work twice for few
+  // points of each (isotropic, two-phase and tile: 58x400x400 with 11 points a
+  // face 3.17, 3.58; 30x300x300 with 7 1.49, 1.73; 64x400x400 with 21 3.69, 3.55).
+  // So for two rows of tiles between two y faces (300x16x300 with 7 points 0.57,
+  // 0.61), and where more than a quarter of the tiles' rows are empty (300x9x300
+  // 0.23, 0.28).  One body covers it: 58x200x200 1.34, 1.21; two 300x9x200 0.41, 0.36.
+  if (!visco && ((d.ni <= 64 && d.pml_on[0] && d.pml_on[1] &&
+                  d.pml_layers[0] + d.pml_layers[1] + 2 < 32) ||
+                 (d.nj <= 16 && d.pml_on[2] && d.pml_on[3]) ||
+                 4 * d.nj < 3 * ((d.nj + 7) / 8 * 8)))
+    return false;
+  // Few blocks: of 512 places (two blocks a compute unit, one with four Maxwell
+  // bodies) each block is a chain of latencies, which the two-phase kernel's
+  // smaller blocks hide better; the more operands a point has, the sooner the
+  // tile's saving of loads outweighs that.  us a step, two-phase and tile, by
+  // blocks: isotropic 856 218, 241; 1456 237, 243; 2214 321, 319; 2496 429, 397;
+  // 2996 484, 438; anisotropic 608 209, 221; 1088 252, 262; 1566 301, 285; one
+  // body 988 273, 280; 1376 389, 364; two 376 202, 215; 640 254, 251; three 288
+  // 214, 227; 448 284, 243; four 352 240, 280; 784 385, 372.
+  const long blocks = (d.ni + 63) / 64 * (long)((d.nj + 7) / 8) * (d.free_top ? d.nk - 4 : d.nk);
+  const long least = visco ? (d.nmaxwell == 1 ? 1152 : (d.nmaxwell < 4 ? 512 : 640))
+                     : d.medium_type == CGFDH_MEDIUM_ELASTIC_ANISO ? 1536 : 2400;
+  return blocks >= least;
 }
 
 // the place in a device volume of a point of the reference's array
@@ -414,7 +459,7 @@ extern "C" int cgfdh_create(const cgfdh_desc* d, cgfdh_solver** out)
     bad = alloc_all(false);
   }
   s->tile = tile_chosen(s);
-  // default stage kernel: where the tile kernel does not step, the anisotropic
+  // default stage kernel: where variant 16 has the two-phase kernel, the anisotropic
   // medium's best is the whole-row kernel through LDS (400x400x200: 11.96 ms a
   // step, the two-phase kernel 12.25)
   s->variant = d->medium_type == CGFDH_MEDIUM_ELASTIC_ANISO && !s->tile ? 18 : 16;
@@ -1172,7 +1217,7 @@ static LaunchCtx make_ctx(const cgfdh_solver* s, hipStream_t stream)
   }
   L.shell_stream = stream;
   L.slab_only = 0;
-  L.bytes = (long)(4 * s->nw + 10 + s->ncmp) * s->vol * (long)sizeof(float);
+  L.bytes = vol_bytes(s);
   return L;
 }
 
@@ -3332,8 +3377,8 @@ extern "C" int cgfdh_batch_autotune(cgfdh_batch* b, int it0)
                                       : std::vector<int>{4, 6, 7, 8, 12, 14, 16, 18};
     if (iso) variants.push_back(3);
     // variant 16 on both of its kernels, where the tile kernel reaches
-    const bool tile = s->tile;
-    bool bt = tile;
+    const bool tile = tile_reaches(s);
+    bool bt = s->tile;
     if (tile) variants.push_back(TWO_PHASE);
     const int groups[][2] = {{9, 2}, {3, 4}, {9, 8}};
     float best = 1e30f;

@@ -19,8 +19,9 @@
 // plane kernel (64x8) with the same phased loads plus the shell; 15 variant
 // 12 compiled for 3 waves per SIMD (a few registers spill) plus the shell;
 // 16 whole rows with the PML faces folded in, the free-surface rows on the
-// general kernel: the tile kernel (stage_tile.h) steps, the two-phase kernel
-// evaluates a single right-hand side and serves volumes past 32-bit offsets; 17 the two-phase interior kernel
+// general kernel: the tile kernel (stage_tile.h) steps, or on grids where it does
+// not pay the two-phase kernel, which also evaluates a single right-hand side;
+// 17 the two-phase interior kernel
 // on the tiles clear of every PML face and the phased shell kernel on the
 // PML slabs (x edges in whole 64-point tiles, y and z slabs in whole rows),
 // free-surface rows on the general kernel.

@@ -1,4 +1,5 @@
-// stage_tile.h -- the default stage kernel (variant 16) of every medium: one
+// stage_tile.h -- the default stage kernel (variant 16) of every medium on all but
+// small grids: one
 // 64 x 8 tile of one plane per block, over whole rows, the PML faces folded in.
 //
 // What bounded the per-point kernels before it (whole rows, two-phase loads)
@@ -436,7 +437,7 @@ void launch_tile_kind(const LaunchCtx& L, const StageParams& P, int kind, int co
 
 // A solver whose arrays fit the 256 MB last-level cache finds them there at
 // the next stage and keeps to plain accesses (100x100x60: 0.291 ms a step
-// against 0.333 non-temporal); a larger one streams past the caches, which
+// against 0.333 non-temporal; the two-phase kernel, chosen there, 0.284); a larger one streams past the caches, which
 // keep the planes and halo rows that neighbours share (600x600x300: 23.3
 // against 23.7, without PML 19.4 against 20.1).
 template <int MT, int NB>

@@ -536,16 +536,17 @@ int cgfdh_last_timing(cgfdh_solver *s, double *run_ms, double *stage_ms,
  * compiled for 3 waves per SIMD; 2..15 run the per-point kernel on the PML
  * and free-surface shell; 16 = plane tiles of 64x8 points over whole rows,
  * operands through LDS, with the PML faces folded in (free-surface rows on the
- * per-point kernel; volumes above 536 M points, cgfdh_onestage and the fused
- * batch cycle on the two-phase kernel over whole rows); 17 = the
+ * per-point kernel; small grids, narrow ones with PML on both x faces, volumes
+ * above 536 M points, cgfdh_onestage and the fused batch cycle on the
+ * two-phase kernel over whole rows); 17 = the
  * two-phase interior kernel on the tiles clear of every PML face plus a
  * shell kernel that requests each PML slab's memory variables first; 18 =
  * the two-phase kernel over whole rows with the metric, medium, slowness and
  * RK combine inputs loaded straight to LDS (global_load_lds), so the stencil
  * values alone hold registers and four waves fit per SIMD.
- * Default 16; 18 for anisotropic volumes above 536 M points.  The environment's
- * CGFDH_TILE=0, read by cgfdh_create, has variant 16 step on the two-phase
- * kernel at every size.
+ * Default 16; for anisotropic grids where that is the two-phase kernel, 18.  The
+ * environment's CGFDH_TILE, read by cgfdh_create, has variant 16 step on the
+ * two-phase kernel at every size (0), or on the tiles wherever they reach (1).
  * Variants 1..3 exist for the isotropic medium only; the visco-elastic
  * medium has 0, 4, 5, 8..11 and 16.
  * All variants produce identical bits. */

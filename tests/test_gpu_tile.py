@@ -15,6 +15,12 @@ SHAPES = [(8, 9, 12), (63, 8, 10), (64, 15, 9), (65, 17, 11), (90, 16, 13), (130
 MEDIA = ["iso", "vti", "aniso", "visco2", "visco3", "visco4"]
 
 
+@pytest.fixture(autouse=True)
+def tiles_at_every_size(monkeypatch):
+    """Small grids step on the two-phase kernel otherwise."""
+    monkeypatch.setenv("CGFDH_TILE", "1")
+
+
 def _case(medium, ni, nj, nk, free, layers):
     pml = (1, 1, 1, 1, 1, 0 if free else 1)
     kind = "visco" if medium.startswith("visco") else medium
@@ -53,13 +59,45 @@ def test_two_phase_steps_match_oracle(ni, nj, nk, medium, monkeypatch):
     test_tile_edges_match_oracle(ni, nj, nk, medium)
 
 
-@pytest.mark.parametrize("medium,nk,variant", [("iso", 500, 16), ("iso", 520, 16),
-                                               ("aniso", 490, 16), ("aniso", 520, 18)])
-def test_default_past_the_tile_kernel(medium, nk, variant):
-    """1024 x 1024 rows and planes of 506, 526 and 496: 531, 552 and 520 M points,
-    either side of two volumes and a plane of 2^32 bytes (537 M)."""
+@pytest.mark.parametrize("gauss", [False, True])
+@pytest.mark.parametrize("medium", ["iso", "vti", "aniso", "visco"])
+def test_tile_run_with_sources_matches_oracle(medium, gauss):
+    from tests.test_gpu_parity import test_run_matches_oracle
+    test_run_matches_oracle(medium, 16, gauss)
+
+
+@pytest.mark.parametrize("medium", ["iso", "visco"])
+def test_tile_run_with_dd_sources_matches_oracle(medium):
+    from tests.test_gpu_dd import test_dd_run_matches_oracle
+    test_dd_run_matches_oracle(medium, 16)
+
+
+def test_tile_steps_in_a_captured_batch():
+    from tests import test_gpu_batch as tb
+    tb.test_batch_matches_oracle()
+    tb.test_batch_equals_individual_runs()
+
+
+# which kernel variant 16 steps on, as the anisotropic medium's default shows it
+# (18 instead of the two-phase kernel): blocks of 64 x 8 points either side of
+# 1536, one tile between two x faces and two tiles between two y faces, rows of
+# tiles that are mostly empty, 1024 x 1024 rows and planes of 506, 526 and 496
+# (531, 552 and 520 M points) either side of two volumes and a plane of 2^32 bytes
+# (537 M)
+@pytest.mark.parametrize("medium,ni,nj,nk,x,y,variant", [
+    ("aniso", 64, 64, 100, 0, 0, 18), ("aniso", 100, 100, 63, 0, 0, 18),
+    ("aniso", 100, 100, 64, 0, 0, 16), ("aniso", 58, 200, 200, 10, 0, 18),
+    ("aniso", 58, 200, 200, 15, 0, 16), ("aniso", 65, 200, 200, 10, 0, 16),
+    ("aniso", 58, 200, 200, 0, 10, 16), ("aniso", 300, 16, 300, 0, 6, 18),
+    ("aniso", 300, 16, 300, 6, 0, 16), ("aniso", 300, 18, 300, 0, 6, 16),
+    ("aniso", 300, 11, 300, 0, 0, 18), ("aniso", 300, 12, 300, 0, 0, 16),
+    ("aniso", 1018, 1018, 490, 0, 0, 16), ("aniso", 1018, 1018, 520, 0, 0, 18),
+    ("iso", 1018, 1018, 500, 0, 0, 16), ("iso", 1018, 1018, 520, 0, 0, 16)])
+def test_default_by_size(medium, ni, nj, nk, x, y, variant, monkeypatch):
     from cgfd3d_amd import MEDIUM_ELASTIC_ANISO, MEDIUM_ELASTIC_ISO, Solver
-    s = Solver(1018, 1018, nk, 0.004, 1, medium_type=MEDIUM_ELASTIC_ANISO if medium == "aniso"
-               else MEDIUM_ELASTIC_ISO)
+    monkeypatch.delenv("CGFDH_TILE")
+    layers = (x, x, y, y, 0, 0)
+    s = Solver(ni, nj, nk, 0.004, 1, pml_on=[n > 0 for n in layers], pml_layers=layers,
+               medium_type=MEDIUM_ELASTIC_ANISO if medium == "aniso" else MEDIUM_ELASTIC_ISO)
     assert s.kernel_choice()[0] == variant
     s.close()
