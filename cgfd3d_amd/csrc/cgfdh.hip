@@ -191,7 +191,8 @@ struct cgfdh_solver {
   // device volumes: rows px apart with the first physical point of each on a
   // 128-byte line, so a wave's 64 points are two lines and neighbouring tiles
   // share none (600x600x300 isotropic: 27.5 against 30.8 ms a step on rows nx
-  // apart); pointers to them are lead floats past the allocation
+  // apart), or where that does not pay nx apart; pointers to them are lead floats
+  // past the allocation
   int px, lead;
   long ss, vol;                  // device plane and volume, in floats
   std::vector<void*> vols;       // their allocations
@@ -368,6 +369,25 @@ static bool tile_chosen(const cgfdh_solver* s)
   return blocks >= least;
 }
 
+// Whether the rows of the volumes start on cache lines, which costs up to 31
+// points a row; the layout to judge is set, with s->px.  CGFDH_PAD=0 or 1, a tuning
+// knob read at creation, decides instead.
+static bool pad_rows(const cgfdh_solver* s)
+{
+  const char* e = getenv("CGFDH_PAD");
+  if (e && (e[0] == '0' || e[0] == '1')) return e[0] == '1';
+  if (s->px == s->nx) return true;
+  // the two-phase kernel gains a hundredth from whole lines and loses more where
+  // they cost it the cache: 100x100x60 isotropic 0.247 ms a step packed, 0.244
+  // padded; 130x90x70 (198 MB and 233) 0.317, 0.350
+  if (!tile_chosen(s)) return false;
+  // nor the tile kernel where the arrays fit the cache without the padding only,
+  // or nearly half of a row were padding: 100x100x100 isotropic (238 MB and 288)
+  // 0.395, 0.426; 10x300x300 0.56 two-phase, 0.75
+  const long padded = vol_bytes(s), packed = padded / s->px * s->nx;
+  return 5 * s->px < 9 * s->nx && !(packed <= LLC && padded > LLC / 8 * 7);
+}
+
 // the place in a device volume of a point of the reference's array
 static long dev_index(const cgfdh_solver* s, long p)
 {
@@ -448,8 +468,10 @@ extern "C" int cgfdh_create(const cgfdh_desc* d, cgfdh_solver** out)
     }
     return bad;
   };
-  int bad = alloc_all(true);
-  if (bad) {
+  set_layout(s, true);
+  const bool pad = pad_rows(s);
+  int bad = alloc_all(pad);
+  if (bad && pad) {
     // a grid that only fits without the rows' padding
     (void)hipGetLastError();
     free_all(s);

@@ -546,7 +546,9 @@ int cgfdh_last_timing(cgfdh_solver *s, double *run_ms, double *stage_ms,
  * values alone hold registers and four waves fit per SIMD.
  * Default 16; for anisotropic grids where that is the two-phase kernel, 18.  The
  * environment's CGFDH_TILE, read by cgfdh_create, has variant 16 step on the
- * two-phase kernel at every size (0), or on the tiles wherever they reach (1).
+ * two-phase kernel at every size (0), or on the tiles wherever they reach (1);
+ * CGFDH_PAD, read there too, decides whether the rows on the device are padded
+ * to cache lines (1) or not (0).
  * Variants 1..3 exist for the isotropic medium only; the visco-elastic
  * medium has 0, 4, 5, 8..11 and 16.
  * All variants produce identical bits. */

@@ -59,6 +59,16 @@ def test_two_phase_steps_match_oracle(ni, nj, nk, medium, monkeypatch):
     test_tile_edges_match_oracle(ni, nj, nk, medium)
 
 
+@pytest.mark.parametrize("pad", ["0", "1"])
+@pytest.mark.parametrize("tile", ["0", "1"])
+@pytest.mark.parametrize("medium", MEDIA)
+def test_packed_and_padded_rows_match_oracle(medium, tile, pad, monkeypatch):
+    monkeypatch.setenv("CGFDH_TILE", tile)
+    monkeypatch.setenv("CGFDH_PAD", pad)
+    for shape in SHAPES[2::3]:
+        test_tile_edges_match_oracle(*shape, medium)
+
+
 @pytest.mark.parametrize("gauss", [False, True])
 @pytest.mark.parametrize("medium", ["iso", "vti", "aniso", "visco"])
 def test_tile_run_with_sources_matches_oracle(medium, gauss):
@@ -101,3 +111,26 @@ def test_default_by_size(medium, ni, nj, nk, x, y, variant, monkeypatch):
                medium_type=MEDIUM_ELASTIC_ANISO if medium == "aniso" else MEDIUM_ELASTIC_ISO)
     assert s.kernel_choice()[0] == variant
     s.close()
+
+
+# 16-point rows, which whole lines would double, and volumes of one Maxwell body
+# that fit the last-level cache without padding only (212 and 256 MB): packed; rows
+# of a line's length and large grids: on whole lines
+@pytest.mark.parametrize("ni,nj,nk,nmaxwell,padded", [
+    (10, 300, 300, 0, False), (100, 100, 60, 1, False), (100, 100, 60, 0, False),
+    (122, 122, 60, 0, True), (100, 150, 150, 0, True)])
+def test_device_memory_of_a_solver(ni, nj, nk, nmaxwell, padded, monkeypatch):
+    import torch
+    from cgfd3d_amd import MEDIUM_ELASTIC_ISO, MEDIUM_VISCO_ISO, Solver
+    monkeypatch.delenv("CGFDH_TILE")
+    Solver(8, 8, 8, 0.004, 1).close()          # code objects, static buffers
+    free = torch.cuda.mem_get_info()[0]
+    s = Solver(ni, nj, nk, 0.004, 1, free_top=False, nmaxwell=nmaxwell,
+               medium_type=MEDIUM_VISCO_ISO if nmaxwell else MEDIUM_ELASTIC_ISO)
+    used = free - torch.cuda.mem_get_info()[0]
+    s.close()
+    px = -(-(ni + 6) // 32) * 32 if padded else ni + 6
+    vols = 4 * (9 + 6 * nmaxwell) + 10 + 3 + 2 * nmaxwell
+    want = 4 * px * (nj + 6) * (vols * (nk + 6) + 36)
+    # allocations are rounded to 2 MB, streams have queues
+    assert want <= used <= want + 2 ** 25
