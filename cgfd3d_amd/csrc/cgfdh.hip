@@ -196,8 +196,8 @@ struct cgfdh_solver {
   int px, lead;
   long ss, vol;                  // device plane and volume, in floats
   std::vector<void*> vols;       // their allocations
-  float* stage = nullptr;        // host rows on their way to and from them
-  size_t stage_n = 0;
+  int dev = 0;
+  long pad_bytes = 0;            // of the rows' padding, held in the device's RowPool
   int ni1, ni2, nj1, nj2, nk1, nk2;
   hipStream_t stream = nullptr;
   hipStream_t stream2 = nullptr; // shell boxes, when they run beside the interior
@@ -293,7 +293,7 @@ static void free_all(cgfdh_solver* s)
 {
   auto F = [](void* p) { if (p) (void)hipFree(p); };
   for (void* v : s->vols) F(v);
-  F(s->mats); F(s->stage);
+  F(s->mats);
   for (auto& f : s->face) {
     F(f.A); F(f.B); F(f.D);
     for (auto& a : f.aux) F(a);
@@ -313,6 +313,62 @@ static void set_layout(cgfdh_solver* s, bool aligned)
   s->px = aligned ? (s->nx + 31) / 32 * 32 : s->nx;
   s->ss = (long)s->px * s->ny;
   s->vol = s->ss * s->nz;
+}
+
+// What the solvers of a device with padded rows share: the buffer that host rows
+// pass on their way to and from the volumes, held by one call at a time and given
+// back with the last of them, and the count of their padding.
+struct RowPool {
+  std::mutex m;
+  float* stage = nullptr;
+  size_t n = 0;
+  int users = 0;
+  long pad_bytes = 0;
+};
+
+static RowPool& row_pool(int dev)
+{
+  static RowPool pools[64];
+  return pools[dev & 63];
+}
+
+// the solver's part in the pool of its device; false without the memory for it,
+// or where all padding together would take more than a sixteenth of the card
+static bool row_pool_join(cgfdh_solver* s, long pad_bytes, size_t total)
+{
+  const long cap = 1l << 24;     // 64 MB
+  // ten volumes, the metric's, at once where they fit; a row of surface matrices
+  const size_t n = std::max(std::min(cap, 10l * s->nx * s->ny * s->nz), 9l * s->nx);
+  RowPool& p = row_pool(s->dev);
+  std::lock_guard<std::mutex> lock(p.m);
+  if (p.pad_bytes + pad_bytes > (long)(total / 16)) return false;
+  if (p.n < n) {
+    float* q = nullptr;
+    if (hipMalloc((void**)&q, n * sizeof(float)) != hipSuccess) {
+      (void)hipGetLastError();
+      return false;
+    }
+    if (p.stage) (void)hipFree(p.stage);
+    p.stage = q;
+    p.n = n;
+  }
+  p.users++;
+  p.pad_bytes += pad_bytes;
+  s->pad_bytes = pad_bytes;
+  return true;
+}
+
+static void row_pool_leave(cgfdh_solver* s)
+{
+  if (!s->pad_bytes) return;
+  RowPool& p = row_pool(s->dev);
+  std::lock_guard<std::mutex> lock(p.m);
+  p.pad_bytes -= s->pad_bytes;
+  s->pad_bytes = 0;
+  if (--p.users) return;
+  if (p.stage) (void)hipFree(p.stage);
+  p.stage = nullptr;
+  p.n = 0;
 }
 
 // of the device volumes: the wavefield's four levels, the metric, the medium
@@ -468,12 +524,19 @@ extern "C" int cgfdh_create(const cgfdh_desc* d, cgfdh_solver** out)
     }
     return bad;
   };
+  // Padding takes no memory that is wanted: at most a sixteenth of the card for all
+  // solvers together, and only where an eighth of the card is left for what the
+  // setters and other solvers allocate.
+  size_t left = 0, total = 0;
+  int bad = hipGetDevice(&s->dev) != hipSuccess || hipMemGetInfo(&left, &total) != hipSuccess;
   set_layout(s, true);
-  const bool pad = pad_rows(s);
-  int bad = alloc_all(pad);
-  if (bad && pad) {
-    // a grid that only fits without the rows' padding
+  const long pad_bytes = vol_bytes(s) / s->px * (s->px - s->nx);
+  bool pad = !bad && pad_rows(s) && (!pad_bytes || row_pool_join(s, pad_bytes, total));
+  if (!bad) bad = alloc_all(pad);
+  if (pad && (bad || (pad_bytes && (hipMemGetInfo(&left, &total) != hipSuccess ||
+                                    left < total / 8)))) {
     (void)hipGetLastError();
+    row_pool_leave(s);
     free_all(s);
     s->vols.clear();
     s->mats = s->pg = nullptr;
@@ -494,6 +557,7 @@ extern "C" int cgfdh_create(const cgfdh_desc* d, cgfdh_solver** out)
                hipEventCreate(&s->ev_run[1]) != hipSuccess))
     bad = 1;
   if (bad) {
+    row_pool_leave(s);
     free_all(s);
     delete s;
     return fail(CGFDH_ENOMEM, "cgfdh_create: device allocation failed for %dx%dx%d", d->ni,
@@ -519,6 +583,7 @@ extern "C" int cgfdh_destroy(cgfdh_solver* s)
     }
     (void)hipStreamDestroy(s->copy_stream);
   }
+  row_pool_leave(s);
   free_all(s);
   for (auto e : s->ev_stage) (void)hipEventDestroy(e);
   (void)hipEventDestroy(s->ev_run[0]);
@@ -562,8 +627,8 @@ __global__ void __launch_bounds__(256) pack_rows_kernel(const float* __restrict_
   }
 }
 
-// host rows to device rows and back, through a staging buffer of at most 64 MB
-// that stays with the solver (a strided host copy would go row by row)
+// host rows to device rows and back, through the pool's buffer (a strided host copy
+// would go row by row)
 static int copy_rows(cgfdh_solver* s, float* dev, int per, float* host, long nrow, bool to_dev)
 {
   const int len = s->nx * per;
@@ -576,36 +641,31 @@ static int copy_rows(cgfdh_solver* s, float* dev, int per, float* host, long nro
     HIPCHK(hipStreamSynchronize(s->stream));
     return CGFDH_OK;
   }
-  const long cap = 1l << 24;
-  const long rows = std::max(1l, std::min(nrow, cap / len));
-  if (s->stage_n < (size_t)(rows * len)) {
-    HIPCHK(hipStreamSynchronize(s->stream));
-    if (s->stage) HIPCHK(hipFree(s->stage));
-    s->stage = nullptr;
-    s->stage_n = 0;
-    // room for the ten volumes of the metric at once, so that a small solver's
-    // setters do not grow it one after another
-    const long n = std::max(rows * len, std::min(cap, 10l * s->nx * s->ny * s->nz));
-    HIPCHK(hipMalloc((void**)&s->stage, n * sizeof(float)));
-    s->stage_n = n;
-  }
-  for (long r = 0; r < nrow; r += rows) {
+  RowPool& p = row_pool(s->dev);
+  std::lock_guard<std::mutex> lock(p.m);
+  const long rows = std::min(nrow, (long)p.n / len);
+  hipError_t e = hipSuccess;
+  for (long r = 0; r < nrow && e == hipSuccess; r += rows) {
     const long n = std::min(rows, nrow - r);
     const size_t bytes = n * len * sizeof(float);
     const dim3 grd((unsigned)std::min(8192l, (n * len + 255) / 256));
     if (to_dev) {
-      HIPCHK(hipMemcpyAsync(s->stage, host + r * len, bytes, hipMemcpyHostToDevice, s->stream));
-      hipLaunchKernelGGL(spread_rows_kernel, grd, dim3(256), 0, s->stream, s->stage,
+      e = hipMemcpyAsync(p.stage, host + r * len, bytes, hipMemcpyHostToDevice, s->stream);
+      if (e != hipSuccess) break;
+      hipLaunchKernelGGL(spread_rows_kernel, grd, dim3(256), 0, s->stream, p.stage,
                          dev + r * pitch, len, pitch, n);
-      HIPCHK(hipGetLastError());
+      e = hipGetLastError();
     } else {
-      hipLaunchKernelGGL(pack_rows_kernel, grd, dim3(256), 0, s->stream, dev + r * pitch,
-                         s->stage, len, pitch, n);
-      HIPCHK(hipGetLastError());
-      HIPCHK(hipMemcpyAsync(host + r * len, s->stage, bytes, hipMemcpyDeviceToHost, s->stream));
+      hipLaunchKernelGGL(pack_rows_kernel, grd, dim3(256), 0, s->stream, dev + r * pitch, p.stage,
+                         len, pitch, n);
+      e = hipGetLastError();
+      if (e != hipSuccess) break;
+      e = hipMemcpyAsync(host + r * len, p.stage, bytes, hipMemcpyDeviceToHost, s->stream);
     }
   }
-  HIPCHK(hipStreamSynchronize(s->stream));
+  // nothing of this call uses the buffer once the lock is given up
+  const hipError_t e2 = hipStreamSynchronize(s->stream);
+  HIPCHK(e != hipSuccess ? e : e2);
   return CGFDH_OK;
 }
 

@@ -548,7 +548,8 @@ int cgfdh_last_timing(cgfdh_solver *s, double *run_ms, double *stage_ms,
  * environment's CGFDH_TILE, read by cgfdh_create, has variant 16 step on the
  * two-phase kernel at every size (0), or on the tiles wherever they reach (1);
  * CGFDH_PAD, read there too, decides whether the rows on the device are padded
- * to cache lines (1) or not (0).
+ * to cache lines (1) or not (0).  All padding together takes a sixteenth of the
+ * card at most, and none where less than an eighth of the card would be left.
  * Variants 1..3 exist for the isotropic medium only; the visco-elastic
  * medium has 0, 4, 5, 8..11 and 16.
  * All variants produce identical bits. */

@@ -132,5 +132,5 @@ def test_device_memory_of_a_solver(ni, nj, nk, nmaxwell, padded, monkeypatch):
     px = -(-(ni + 6) // 32) * 32 if padded else ni + 6
     vols = 4 * (9 + 6 * nmaxwell) + 10 + 3 + 2 * nmaxwell
     want = 4 * px * (nj + 6) * (vols * (nk + 6) + 36)
-    # allocations are rounded to 2 MB, streams have queues
-    assert want <= used <= want + 2 ** 25
+    # allocations are rounded to 2 MB, streams have queues, padded rows a 64 MB buffer
+    assert want <= used <= want + 2 ** 25 + (2 ** 26 if px != ni + 6 else 0)
