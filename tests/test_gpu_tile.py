@@ -34,9 +34,12 @@ def _case(medium, ni, nj, nk, free, layers):
 @pytest.mark.parametrize("medium", MEDIA)
 @pytest.mark.parametrize("ni,nj,nk", SHAPES)
 def test_tile_edges_match_oracle(ni, nj, nk, medium):
-    nt, dt = 9, 0.004
     free = (ni + nk) % 2 == 0
-    case = _case(medium, ni, nj, nk, free, 5 if ni < 60 else 3)
+    _match(_case(medium, ni, nj, nk, free, 5 if ni < 60 else 3), 9)
+
+
+def _match(case, nt):
+    dt = 0.004
     w, aux = cs.random_wavefield(case, seed=3).reshape(-1), cs.random_aux(case, seed=3)
     orc = po.Oracle(case)
     w_o, a_o, _ = orc.run(dt, nt, w=w, aux=aux)
@@ -49,6 +52,23 @@ def test_tile_edges_match_oracle(ni, nj, nk, medium):
     assert np.isfinite(w_o).all() and np.abs(w_o).max() > 0
     assert np.array_equal(w_g, np.asarray(w_o).reshape(-1))
     assert np.array_equal(a_g, np.asarray(a_o).reshape(-1))
+
+
+# volumes just past the last-level cache, 256 MB, on which the kernel's accesses
+# that no other point repeats are non-temporal, in 5 to 10 units of planes, the last
+# one short
+@pytest.mark.parametrize("medium,ni,nj,nk", [
+    ("iso", 122, 100, 98), ("vti", 122, 100, 93), ("aniso", 122, 100, 71), ("visco2", 90, 90, 71),
+    ("visco3", 90, 90, 55), ("visco4", 90, 90, 45)])
+def test_large_volumes_match_oracle(medium, ni, nj, nk):
+    case = _case(medium, ni, nj, nk, True, 7)
+    nw = cs.ncomp(case)
+    ncoef = 10 + len(case["med"])
+    assert 4 * (4 * nw + ncoef) * (-(-(ni + 6) // 32) * 32) * (nj + 6) * (nk + 6) > 2 ** 28
+    planes = nk - 4
+    chunk = -(-planes // (planes // 8))
+    assert planes // 8 >= 5 and planes % chunk != 0
+    _match(case, 2)
 
 
 @pytest.mark.parametrize("medium", MEDIA)
