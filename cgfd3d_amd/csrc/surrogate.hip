@@ -78,9 +78,17 @@ struct GemmArgs {
 // row tiles or splits would leave XCDs idle and stay in plain order.
 enum { ORD_PLAIN = 0, ORD_ROWS = 1, ORD_SPLIT = 2 };
 
+// a launch holds below 2^32 threads in x: more blocks than these go on in y
+constexpr unsigned GRID_X = 1u << 20;
+
+static dim3 gemm_grid(long blocks)
+{
+  return dim3((unsigned)std::min(blocks, (long)GRID_X), (unsigned)((blocks + GRID_X - 1) / GRID_X));
+}
+
 __device__ __forceinline__ bool gemm_tile(const GemmArgs& g, int& x, int& y, int& z)
 {
-  const unsigned f = blockIdx.x, q = f / 8, xcd = f % 8;
+  const unsigned f = blockIdx.y * GRID_X + blockIdx.x, q = f / 8, xcd = f % 8;
   if (g.order == ORD_ROWS) {
     x = q / g.nt * 8 + xcd;
     y = q % g.nt;
@@ -424,9 +432,10 @@ __global__ __launch_bounds__(256) void splitk_reduce_kernel(int S, int M, int N,
 static void launch_reduce(hipStream_t st, int S, int M, int N, const float* work, float* out,
                           long ldo, float* csum)
 {
+  const long n = (long)M * N + (csum ? N : 0), outs = N % 4 == 0 ? n / 4 : n;
   int G = 1;
-  while (G < 32 && G * 4 <= S) G *= 2;
-  const long n = (long)M * N + (csum ? N : 0), L = 256 / G;
+  while (G < 32 && G * 4 <= S && outs * G * 2 < 1l << 31) G *= 2;   // a launch's threads
+  const long L = 256 / G;
   if (N % 4 == 0)
     hipLaunchKernelGGL(splitk_reduce_kernel<4>, dim3((unsigned)((n / 4 + L - 1) / L)), dim3(256),
                        0, st, S, M, N, G, work, out, ldo, csum);
@@ -695,7 +704,7 @@ static int gemm_launch(const char* name, GemmArgs g, int transA, int transB, int
     if (wide) return;
     blocks = shape(BM, BN);
     if (blocks > 0x7fffffffl) return;
-    const dim3 grid((unsigned)blocks), blk(128 * WM);
+    const dim3 grid = gemm_grid(blocks), blk(128 * WM);
     switch (form) {
     case 0: hipLaunchKernelGGL((gemm_bf16_kernel<0, 0, BM, BN, BK, NS, WM, 2>), grid, blk, 0, st, g); break;
     case 1: hipLaunchKernelGGL((gemm_bf16_kernel<0, 1, BM, BN, BK, NS, WM, 2>), grid, blk, 0, st, g); break;
@@ -722,7 +731,8 @@ static int gemm_launch(const char* name, GemmArgs g, int transA, int transB, int
     wide = too_wide(CGFDS_I(64), CGFDS_I(128), CGFDS_I(64));
     if (!wide) {
       blocks = shape(64, 128);
-      hipLaunchKernelGGL((gemm_bf16_kernel<0, 0, 64, 128, 64, 3, 2, 2>), dim3((unsigned)blocks),
+      if (blocks > 0x7fffffffl) return bad("more than 2^31 - 1 tiles");
+      hipLaunchKernelGGL((gemm_bf16_kernel<0, 0, 64, 128, 64, 3, 2, 2>), gemm_grid(blocks),
                          dim3(256), 0, st, g);
     }
   } else if (mid >= 256) {
@@ -733,7 +743,7 @@ static int gemm_launch(const char* name, GemmArgs g, int transA, int transB, int
   if (wide) {
     // one tile serves them: matrices of gigabytes of which few values are read
     blocks = g.y ? shape(64, 128) : shape(64, 32);
-    const dim3 grid((unsigned)blocks), blk(256);
+    const dim3 grid = gemm_grid(blocks), blk(256);
 #define CGFDS_W(TA, TB) \
   hipLaunchKernelGGL((gemm_bf16_kernel<TA, TB, 64, 32, 128, 4, 2, 2, true>), grid, blk, 0, st, g)
     if (blocks > 0x7fffffffl) return bad("more than 2^31 - 1 tiles");

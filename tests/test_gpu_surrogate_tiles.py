@@ -122,6 +122,27 @@ def test_rows_past_32_bit_offsets(M, N, K, transA, transB, lda, ldb):
         assert ((s.double().cpu() - g.sum(0)).abs() <= K * 2.0 ** -23 * g.abs().sum(0)).all()
 
 
+def test_more_blocks_than_a_launch_holds_in_x():
+    """2^27 rows in 8 splits: 2^23 blocks of 512 threads.  Rows of ones among zeros,
+    so that the result is small whole numbers."""
+    from cgfd3d_amd import surrogate as sg
+    M, N, K, S = 1 << 27, 8, 256, 8
+    a = torch.zeros((M, K), dtype=torch.bfloat16, device="cuda:0")
+    at = [0, 127, 128, 1 << 26, M - 129, M - 1]
+    a[at] = 1
+    b = torch.zeros((K, N), dtype=torch.bfloat16, device="cuda:0")
+    b[::3] = 1
+    b[1, 5] = 2
+    c = torch.empty((M, N), device="cuda:0")
+    work = torch.empty(S * M * N, device="cuda:0")
+    sg.gemm(M, N, K, a, K, 0, b, N, 0, C32=c, ldc32=N, splitk=S, work=work)
+    want = b.float().sum(0)
+    assert torch.equal(c[at], want.expand(len(at), N))
+    assert int(torch.count_nonzero(c)) == len(at) * N
+    del a, c, work
+    torch.cuda.empty_cache()
+
+
 def test_contraction_of_rows_past_32_bit_offsets():
     from cgfd3d_amd import surrogate as sg
     from cgfd3d_amd._lib import check, lib
