@@ -528,11 +528,13 @@ extern "C" int cgfdh_create(const cgfdh_desc* d, cgfdh_solver** out)
   // solvers together, and only where an eighth of the card is left for what the
   // setters and other solvers allocate.
   size_t left = 0, total = 0;
-  int bad = hipGetDevice(&s->dev) != hipSuccess || hipMemGetInfo(&left, &total) != hipSuccess;
+  const bool known = hipGetDevice(&s->dev) == hipSuccess &&
+                     hipMemGetInfo(&left, &total) == hipSuccess;
   set_layout(s, true);
   const long pad_bytes = vol_bytes(s) / s->px * (s->px - s->nx);
-  bool pad = !bad && pad_rows(s) && (!pad_bytes || row_pool_join(s, pad_bytes, total));
-  if (!bad) bad = alloc_all(pad);
+  const bool pad = pad_rows(s) &&
+                   (!pad_bytes || (known && row_pool_join(s, pad_bytes, total)));
+  int bad = alloc_all(pad);
   if (pad && (bad || (pad_bytes && (hipMemGetInfo(&left, &total) != hipSuccess ||
                                     left < total / 8)))) {
     (void)hipGetLastError();
