@@ -400,28 +400,42 @@ static bool tile_chosen(const cgfdh_solver* s)
   if (!s->lead && vol_bytes(s) > LLC) return false;
   const cgfdh_desc& d = s->d;
   const bool visco = d.medium_type == CGFDH_MEDIUM_VISCO_ISO;
-  // One tile a row that meets both x faces does a tile's face work twice for few
-  // points of each (isotropic, two-phase and tile: 58x400x400 with 11 points a
-  // face 3.17, 3.58; 30x300x300 with 7 1.49, 1.73; 64x400x400 with 21 3.69, 3.55).
-  // So for two rows of tiles between two y faces (300x16x300 with 7 points 0.57,
-  // 0.61), and where more than a quarter of the tiles' rows are empty (300x9x300
-  // 0.23, 0.28).  One body covers it: 58x200x200 1.34, 1.21; two 300x9x200 0.41, 0.36.
-  if (!visco && ((d.ni <= 64 && d.pml_on[0] && d.pml_on[1] &&
-                  d.pml_layers[0] + d.pml_layers[1] + 2 < 32) ||
-                 (d.nj <= 16 && d.pml_on[2] && d.pml_on[3]) ||
-                 4 * d.nj < 3 * ((d.nj + 7) / 8 * 8)))
+  BoxParams b;
+  const int nk = d.free_top ? d.nk - 4 : d.nk;
+  tile_box(d.ni, d.nj, nk, b);
+  const long blocks = (long)b.tiles_x * b.tiles_y * nk;
+  int round = 0;                 // the first XCD's blocks, no other has more
+  for (int u = 0; u < b.tiles_y * b.nchunk && round <= 64; u += 8)
+    round += b.tiles_x * std::min(b.kchunk, nk - u / b.tiles_y * b.kchunk);
+  // Two rows of tiles between two y faces do a tile's face work twice for few points
+  // of each (300x16x300 isotropic, 7 points a face, two-phase and tile, 0.57 and 0.61
+  // ms a step), as tiles with more than a quarter of their rows empty do theirs
+  // (300x9x300 0.23, 0.28).  The visco-elastic medium's other traffic covers it (two
+  // bodies 300x9x200 0.41, 0.36).
+  if (!visco && ((d.nj <= 16 && d.pml_on[2] && d.pml_on[3]) ||
+                 4 * d.nj < 3 * TILE_ROWS * b.tiles_y))
     return false;
-  // Few blocks: of 512 places (two blocks a compute unit, one with four Maxwell
-  // bodies) each block is a chain of latencies, which the two-phase kernel's
+  // One nearly full round of blocks, 64 on an XCD (two a compute unit, one with four
+  // Maxwell bodies): 400 of 90x60x29 isotropic 144 us a step two-phase, 138 on tiles,
+  // anisotropic 157, 149, one body 202, 179; but 442 of 100x100x21, two rounds on
+  // some XCDs, isotropic 144, 163.
+  if (round <= 64 && blocks >= 384 && !(visco && d.nmaxwell == 4)) return true;
+  // One tile a row between two x faces, as above: 58x400x400 with 11 points a face
+  // 3.17, 3.58; 30x300x300 with 7 1.49, 1.73; 64x400x400 with 21 3.69, 3.55; one
+  // body 58x200x200 1.34, 1.21; four, one block a compute unit, 33x55x228 0.75, 0.78,
+  // 39x80x150 0.71, 0.69.
+  if ((!visco || (d.nmaxwell == 4 && d.ni <= 36)) && b.tiles_x == 1 && d.pml_on[0] &&
+      d.pml_on[1] && d.pml_layers[0] + d.pml_layers[1] + 2 < 32)
+    return false;
+  // Few rounds: each block is a chain of latencies, which the two-phase kernel's
   // smaller blocks hide better; the more operands a point has, the sooner the
   // tile's saving of loads outweighs that.  us a step, two-phase and tile, by
   // blocks: isotropic 856 218, 241; 1456 237, 243; 2214 321, 319; 2496 429, 397;
-  // 2996 484, 438; anisotropic 608 209, 221; 1088 252, 262; 1566 301, 285; one
-  // body 988 273, 280; 1376 389, 364; two 376 202, 215; 640 254, 251; three 288
-  // 214, 227; 448 284, 243; four 352 240, 280; 784 385, 372.
-  const long blocks = (d.ni + 63) / 64 * (long)((d.nj + 7) / 8) * (d.free_top ? d.nk - 4 : d.nk);
-  const long least = visco ? (d.nmaxwell == 1 ? 1152 : (d.nmaxwell < 4 ? 512 : 640))
-                     : d.medium_type == CGFDH_MEDIUM_ELASTIC_ANISO ? 1536 : 2400;
+  // 2996 484, 438; anisotropic 608 209, 221; 1088 252, 262; 1380 330, 301; one
+  // body 988 273, 280; 1376 389, 364; two 376 202, 215; 420 221, 195; three 288
+  // 214, 227; 448 284, 243; four 352 240, 280; 512 305, 280.
+  const long least = visco ? (d.nmaxwell == 1 ? 1152 : 400)
+                     : d.medium_type == CGFDH_MEDIUM_ELASTIC_ANISO ? 1344 : 2400;
   return blocks >= least;
 }
 
@@ -439,9 +453,16 @@ static bool pad_rows(const cgfdh_solver* s)
   if (!tile_chosen(s)) return false;
   // nor the tile kernel where the arrays fit the cache without the padding only,
   // or nearly half of a row were padding: 100x100x100 isotropic (238 MB and 288)
-  // 0.395, 0.426; 10x300x300 0.56 two-phase, 0.75
+  // 0.395, 0.426; 10x300x300 0.56 two-phase, 0.75.  A few points a row do not
+  // matter: 209x49x100 isotropic (239 MB and 249) 0.506, 0.479.  The visco-elastic
+  // medium, most of whose arrays a stage reads once, keeps its packed rows a little
+  // past the cache: four bodies 42x86x94 (258 MB and 344) 0.329, 0.409, two 50x90x120
+  // (261, 298) 0.318, 0.355; three 42x86x130 (291, 388) 0.416, 0.402.
   const long padded = vol_bytes(s), packed = padded / s->px * s->nx;
-  return 5 * s->px < 9 * s->nx && !(packed <= LLC && padded > LLC / 8 * 7);
+  const bool visco = s->d.medium_type == CGFDH_MEDIUM_VISCO_ISO;
+  return 5 * s->px < 9 * s->nx &&
+         !(packed <= LLC && padded > LLC / 8 * 7 && 25 * s->px >= 27 * s->nx) &&
+         !(visco && packed <= LLC / 8 * 9 && padded > LLC && 8 * s->px >= 9 * s->nx);
 }
 
 // the place in a device volume of a point of the reference's array

@@ -1,6 +1,6 @@
-// stage_tile.h -- the default stage kernel (variant 16) of every medium on all but
-// small grids: one
-// 64 x 8 tile of one plane per block, over whole rows, the PML faces folded in.
+// stage_tile.h -- the default stage kernel (variant 16) of every medium, on all but
+// small grids: one 64 x 8 tile of one plane per block, over whole rows, the PML
+// faces folded in.
 //
 // What bounded the per-point kernels before it (whole rows, two-phase loads)
 // was the vector memory path of the compute units, not HBM: 165 loads and 18
@@ -15,11 +15,15 @@
 //    variables of the first PML face;
 //  * rows start on 128-byte lines, so a wave's load is two lines, not three;
 //  * registers are kept to 128, 4 waves a SIMD in two blocks a compute unit,
-//    whose loads cover each other's arithmetic.
+//    whose loads cover each other's arithmetic (three Maxwell bodies spill one
+//    register in the middle stages; four take 94 KB of LDS and up to 139
+//    registers: one block a unit, 2 waves a SIMD).
 // 95 vector memory instructions a point are left and 1.14 times the algorithmic
 // traffic (the two-phase kernel: 1.15), 4.7 TB/s on it.  600x600x300 isotropic, ms
 // a step, before and now: 29.7, 23.3; without PML 24.7, 19.4; 400x400x200 VTI
-// 10.1, 8.3; anisotropic 11.8, 9.9; visco-elastic (3 bodies) 22.7, 15.9.
+// 10.1, 8.3; anisotropic 11.8, 9.9; visco-elastic (3 bodies) 22.7, 15.9;
+// 200x200x100 with one to four bodies 2.29, 2.81, 3.34, 3.85 and 1.76, 2.05, 2.43,
+// 2.95.
 #pragma once
 #include <type_traits>
 
@@ -398,20 +402,10 @@ template <int KIND, int MT, int NB, int NT>
 static void launch_tile(const LaunchCtx& L, const StageParams& P, int code)
 {
   constexpr int TY = 8;
+  static_assert(TY == TILE_ROWS, "");
   BoxParams B;
-  const int kmain = L.free_top ? L.nk2 - 4 : L.nk2;
-  memset(&B, 0, sizeof B);
+  const int grid = 8 * tile_box(L.ni, L.nj, L.free_top ? L.nk - 4 : L.nk, B);
   B.i0 = L.ni1; B.j0 = L.nj1; B.k0 = L.nk1;
-  B.ni = L.ni2 - L.ni1 + 1; B.nj = L.nj2 - L.nj1 + 1; B.nk = kmain - L.nk1 + 1;
-  B.tiles_x = (B.ni + 63) / 64;
-  B.tiles_y = (B.nj + TY - 1) / TY;
-  // at least 512 units, 64 an XCD, of no fewer than 8 planes (each re-reads 4):
-  // 600x600x300 isotropic 23.3 ms a step, against 24.9 with units of all planes
-  // and 25.4 with an eighth of the rows to each XCD; 160x160x100 0.85, 0.99
-  B.nchunk = std::max(1, std::min((512 + B.tiles_y - 1) / B.tiles_y, B.nk / 8));
-  B.kchunk = (B.nk + B.nchunk - 1) / B.nchunk;
-  B.nchunk = (B.nk + B.kchunk - 1) / B.kchunk;
-  const int grid = (B.tiles_y * B.nchunk + 7) / 8 * 8 * B.tiles_x * B.kchunk;
   dim3 blk(64, TY, 1);
 #define CGFDH_TI(c, DX, DY, DZ)                                                             \
   case c:                                                                                   \
@@ -454,7 +448,9 @@ void launch_tile_mt(const LaunchCtx& L, const StageParams& P, int kind, int dx, 
 {
   const int code = dx * 4 + dy * 2 + dz;
   if constexpr (MT == MEDIUM_VISCO) {
-    // LDS for three bodies leaves room for two blocks a compute unit
+    // LDS for three bodies leaves room for two blocks a compute unit; fewer pay for
+    // three and are still ahead of the two-phase kernel (200x200x100, one body 1.76
+    // ms a step, 2.19)
     if (P.nmax <= 3)
       launch_tile_nt<MT, 3>(L, P, kind, code);
     else

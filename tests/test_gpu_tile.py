@@ -110,13 +110,14 @@ def test_tile_steps_in_a_captured_batch():
 
 # which kernel variant 16 steps on, as the anisotropic medium's default shows it
 # (18 instead of the two-phase kernel): blocks of 64 x 8 points either side of
-# 1536, one tile between two x faces and two tiles between two y faces, rows of
+# 1344, one round of 480 and 352 of them and two of 494, one tile between two x faces and two tiles between two y faces, rows of
 # tiles that are mostly empty, 1024 x 1024 rows and planes of 506, 526 and 496
 # (531, 552 and 520 M points) either side of two volumes and a plane of 2^32 bytes
 # (537 M)
 @pytest.mark.parametrize("medium,ni,nj,nk,x,y,variant", [
-    ("aniso", 64, 64, 100, 0, 0, 18), ("aniso", 100, 100, 63, 0, 0, 18),
-    ("aniso", 100, 100, 64, 0, 0, 16), ("aniso", 58, 200, 200, 10, 0, 18),
+    ("aniso", 64, 64, 100, 0, 0, 18), ("aniso", 122, 122, 19, 0, 0, 16),
+    ("aniso", 122, 122, 15, 0, 0, 18), ("aniso", 100, 100, 23, 0, 0, 18), ("aniso", 100, 100, 55, 0, 0, 18),
+    ("aniso", 100, 100, 56, 0, 0, 16), ("aniso", 58, 200, 200, 10, 0, 18),
     ("aniso", 58, 200, 200, 15, 0, 16), ("aniso", 65, 200, 200, 10, 0, 16),
     ("aniso", 58, 200, 200, 0, 10, 16), ("aniso", 300, 16, 300, 0, 6, 18),
     ("aniso", 300, 16, 300, 6, 0, 16), ("aniso", 300, 18, 300, 0, 6, 16),
@@ -133,11 +134,13 @@ def test_default_by_size(medium, ni, nj, nk, x, y, variant, monkeypatch):
     s.close()
 
 
-# 16-point rows, which whole lines would double, and volumes of one Maxwell body
-# that fit the last-level cache without padding only (212 and 256 MB): packed; rows
-# of a line's length and large grids: on whole lines
+# 16-point rows, which whole lines would double, volumes of one Maxwell body that fit
+# the last-level cache without padding only (212 and 256 MB) and of two that nearly
+# do (261 and 298): packed; rows of a line's length or nearly, and large grids: on
+# whole lines
 @pytest.mark.parametrize("ni,nj,nk,nmaxwell,padded", [
-    (10, 300, 300, 0, False), (100, 100, 60, 1, False), (100, 100, 60, 0, False),
+    (10, 300, 300, 0, False), (100, 100, 60, 1, False), (50, 90, 120, 2, False),
+    (209, 49, 100, 0, True), (100, 100, 60, 0, False),
     (122, 122, 60, 0, True), (100, 150, 150, 0, True)])
 def test_device_memory_of_a_solver(ni, nj, nk, nmaxwell, padded, monkeypatch):
     import torch
