@@ -436,7 +436,8 @@ def main():
     ap.add_argument("--steps", type=int, default=20)
     ap.add_argument("--warmup", type=int, default=3)
     ap.add_argument("--variant", type=int, default=None,
-                    help="stage kernels (default: 16): 0 per-point, 1 "
+                    help="stage kernels (default: 16, 18 for small anisotropic grids): 0 "
+                         "per-point, 1 "
                          "tiled, 2/3 z-marching interior + "
                          "shell, 4/5 per-point interior (64x4 / 64x2) + shell, 6/7 "
                          "x-vectorised interior (2 / 4 points per thread) + shell, 8/9 "
@@ -445,7 +446,8 @@ def main():
                          "two-phase per-point interior + shell, 13 the same with the RK "
                          "combine loads last, 14 LDS-tiled interior with phased loads + shell, "
                          "15 variant 12 built for 3 waves per SIMD, 16 plane "
-                         "tiles of whole rows through LDS with the PML faces folded in, 17 "
+                         "tiles of whole rows through LDS with the PML faces folded in (small "
+                         "and narrow grids: the whole-row two-phase kernel), 17 "
                          "variant 12 with a two-phase shell, 18 whole-row two-phase kernel with "
                          "the operands that have no stencil loaded straight to LDS; with --workload batch a "
                          "given variant serves every grid and the autotune is skipped")
